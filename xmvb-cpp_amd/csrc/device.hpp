@@ -33,6 +33,10 @@ __device__ __forceinline__ void problem_block(int& x, int& z) {
     x = (int)(k % nx);
 }
 
+// The slot's determinant pairs are evaluated in the string form (strings.hip): the pair kernels of the
+// same launch leave it alone. Uniform over a launch's workgroups of a slot.
+__device__ __forceinline__ bool string_slot(const SlotDesc& sd) { return to_global(sd.flags)[FLAG_STRINGS] != 0; }
+
 // unordered pair t = e(e+1)/2 + d with d <= e
 __device__ __forceinline__ void unpack_pair(long long t, int& d, int& e) {
     long long x = (long long)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);

@@ -177,6 +177,8 @@ struct Lane {
     bool busy = false;
     bool with_grad = false;
     bool events_valid = false;
+    bool strings = false;       // the last forward offered the string form
+    bool pair_kernels = true;   // and launched the pair kernels beside it
     bool scratch = false;  // the launch ran on a workspace outside the slots (no-allocation entry point)
     int ticket = -1;
     std::vector<int> slots;
@@ -212,6 +214,7 @@ struct vbe_pool {
     // forward one-pair-per-lane blocks (the lane-group kernel takes twice this), backward blocks
     int fwd_target = kLaneBlocks;
     int bwd_target = kLaneBlocks;
+    int pair_hold = 0;  // launches left that include the pair kernels from the start (evaluate_now)
 
     // serializes host access to the pool's lanes and slots between the caller's thread and the
     // request scheduler's dispatcher thread
@@ -310,6 +313,58 @@ long long pair_count(const vbe_pool* p) { return (long long)p->topo.n_det * (p->
 
 int bwd_blocks_cap(const vbe_pool* p) {
     return (int)std::min<long long>(kMaxBwdBlocksPerSlot, std::max<long long>(1, (pair_count(p) + 7) / 8));
+}
+
+// Device copies of the string form's tables. The host vectors must outlive the stream's copies.
+void upload_string_tables(const xmvb_amd::StringTables& h, DeviceArena& A, xmvb_amd::StringTopo& d, hipStream_t st) {
+    d = xmvb_amd::StringTopo{};
+    if (!h.enabled) return;
+    auto put = [&](auto& dst, const auto& v) {
+        using E = std::remove_cv_t<std::remove_reference_t<decltype(v[0])>>;
+        E* p = A.alloc<E>(v.size());
+        if (!v.empty()) upload(p, v.data(), v.size(), st);
+        dst = p;
+    };
+    auto space = [&](xmvb_amd::StringSpace& s, const xmvb_amd::StringTables::Space& hs) {
+        s.m = hs.m;
+        s.N = hs.N;
+        s.noff = hs.noff;
+        s.J = hs.J;
+        put(s.mask, hs.mask);
+        put(s.e1, hs.e1);
+    };
+    space(d.a, h.a);
+    space(d.b, h.b);
+    put(d.rank, h.rank);
+    put(d.arank, h.arank);
+    put(d.brank, h.brank);
+    put(d.aoff, h.aoff);
+    put(d.adet, h.adet);
+    put(d.boff, h.boff);
+    put(d.bdet, h.bdet);
+    put(d.soff, h.soff);
+    put(d.slink, h.slink);
+    put(d.goff, h.goff);
+    put(d.glink, h.glink);
+    put(d.wtab, h.wtab);
+    put(d.e2b, h.e2b);
+    put(d.e2a, h.e2a);
+    put(d.w2off_a, h.w2off_a);
+    put(d.w2off_b, h.w2off_b);
+    put(d.w2link_a, h.w2link_a);
+    put(d.w2link_b, h.w2link_b);
+    put(d.alist, h.alist);
+    put(d.order, h.order);
+    put(d.pitem, h.pitem);
+    d.npitem = (int)h.pitem.size();
+    d.nw = h.nw;
+    d.nq_a = h.nq_a;
+    d.nq_b = h.nq_b;
+    d.wchunks = h.wchunks;
+    d.sym = h.sym;
+    d.gchunks = h.gchunks;
+    d.ak = h.ak;
+    d.enabled = 1;
 }
 
 std::unique_ptr<vbe_pool> make_pool(vbe_context* ctx, const vbe_topology_view& t, int n_act, int n_alpha, int n_beta,
@@ -453,6 +508,10 @@ std::unique_ptr<vbe_pool> make_pool(vbe_context* ctx, const vbe_topology_view& t
         if (T.state_idx[k] >= ns)
             throw StatusError(VBE_ERR_ARGUMENT, "selected state " + std::to_string(T.state_idx[k]) +
                                                     " is out of range for " + std::to_string(ns) + " structures");
+    xmvb_amd::StringTables tables =
+        xmvb_amd::build_string_tables(n_act, n_alpha, n_beta, nd, t.alpha_masks, t.det_alpha, t.beta_masks, t.det_beta,
+                                      off.data(), t.term_structure, t.term_coefficient, flip);
+    upload_string_tables(tables, A, T.str, st);
     check(xmvb_amd::configure_kernels(n_act, T.ng, ns, std::max(n_alpha, n_beta)), "hipFuncSetAttribute");
     check(hipStreamSynchronize(st), "hipStreamSynchronize");
     p->slots.resize(capacity);
@@ -473,7 +532,9 @@ void check_slots_free(const vbe_pool* p, const int* slots, int count) {
 // Per-evaluation workspace of one slot of a pool, carved from one block of device memory (arrays
 // aligned to 256 bytes). With base == nullptr nothing is assigned and only the size is returned.
 // The slot's own arena and the no-allocation entry point's static scratch use this same layout.
-size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* base, SlotDesc& d) {
+// The string form's arrays lie over the pair kernels' partial rows where they fit (a slot uses one
+// or the other), else behind everything else; strings = false leaves them out.
+size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* base, SlotDesc& d, bool strings = true) {
     const TopoDesc& T = p->topo;
     const size_t n = T.n, np = T.np, nd = T.n_det, ns = T.n_str;
     size_t off = 0;
@@ -504,7 +565,8 @@ size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* ba
     take(d.dcoef, nd * (size_t)T.n_states);
     take(d.state_energy, (size_t)xmvb_amd::kMaxStates);
     const size_t len = (size_t)T.ng + 2 * n * n;
-    take(d.partials, (size_t)(bwd_blocks_cap(p) + xmvb_amd::kListBlocks + xmvb_amd::kSingularBlocks) * len);
+    const size_t partial_rows = (size_t)(bwd_blocks_cap(p) + xmvb_amd::kListBlocks + xmvb_amd::kSingularBlocks) * len;
+    take(d.partials, partial_rows);
     take(d.dsum, len);
     take(d.dL, (size_t)n_aux * np);
     take(d.gcn, n * n_bf);
@@ -514,6 +576,14 @@ size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* ba
     take(d.singular_flag, (size_t)pair_count(p));
     take(d.chunk_count,
          (size_t)(std::max<long long>(T.n_lane_pairs, pair_count(p)) / xmvb_amd::kCompactChunk + 2));
+    if (base) d.sw = xmvb_amd::StringWork{};
+    if (strings && T.str.enabled) {
+        xmvb_amd::StringWork unused{};
+        const size_t count = xmvb_amd::string_work_carve(T, nullptr, unused);
+        double* work = d.partials;
+        if (count > partial_rows) take(work, count);
+        if (base) (void)xmvb_amd::string_work_carve(T, work, d.sw);
+    }
     return (off + 255) & ~size_t(255);
 }
 
@@ -668,6 +738,12 @@ LaunchShape shape_for(const vbe_pool* p, const std::vector<SlotInput>& in, bool 
             sh.any_flat = true;
         }
     }
+    // A caller that sets its own condition limit asks for the pair kernels (compare them pair by pair
+    // with another program, or force their complete-pivoting path); the default leaves the choice
+    // to each slot's S_act.
+    sh.strings = p->topo.str.enabled && sh.lane_bwd && sh.lane_cond_limit == xmvb_amd::kLaneConditionDefault &&
+                 (p->topo.n_det >= xmvb_amd::kStringDets || (!pinned && count >= xmvb_amd::kStringBatch));
+    for (const auto& x : in) sh.strings = sh.strings && p->slots[x.slot].desc.sw.Sinv;
     sh.davidson = p->eigensolver == VBE_EIGENSOLVER_DAVIDSON;
     if (sh.davidson && (p->topo.n_states > 1 || p->topo.state_idx[0] != 0))
         throw StatusError(VBE_ERR_UNSUPPORTED, "the Davidson eigensolver finds the lowest structure root only; "
@@ -680,15 +756,25 @@ LaunchShape shape_for(const vbe_pool* p, const std::vector<SlotInput>& in, bool 
 
 // Enqueue forward and/or backward for a set of slots on a lane, then the D2H of energies and flags.
 // ws (optional, single-slot launches): a descriptor whose workspace replaces the slot's own.
+// strings_only: where the string form is offered, leave the pair kernels out (see evaluate_now).
 // timed: record the phase events (read by finish into the pool's phase times); the optimiser's
 // inner evaluations skip them, a dozen event records per launch being host time on its critical path.
 void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
-             const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true) {
+             const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true, bool strings_only = false) {
     const int count = (int)in.size();
     if (count <= 0 || count > p->capacity) throw StatusError(VBE_ERR_ARGUMENT, "invalid number of slots");
     if (ws && count != 1) throw StatusError(VBE_ERR_ARGUMENT, "a replacement workspace serves one slot");
     hipStream_t st = lane.stream;
-    const LaunchShape sh = shape_for(p, in, pinned);
+    LaunchShape sh = shape_for(p, in, pinned);
+    if (ws && !ws->sw.Sinv) sh.strings = false;
+    // the gradient of an earlier forward follows the form that forward took
+    if (forward) {
+        lane.strings = sh.strings;
+        lane.pair_kernels = !sh.strings || !strings_only;
+    } else {
+        sh.strings = lane.strings;
+    }
+    sh.pair_kernels = lane.pair_kernels;
     // the side stream only when it is idle: queued behind another lane's launch it would delay this one
     const xmvb_amd::SideStream* side =
         lane.side.st != st && hipStreamQuery(lane.side.st) == hipSuccess ? &lane.side : nullptr;
@@ -793,6 +879,29 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
     if (status != VBE_OK && !slot_status) throw StatusError(status, err);
 }
 
+// A launch that the caller waits for at once: the string form alone first, without the idle launches of the
+// pair kernels (fourteen, 50-60 us of a 510 us evaluation of 252 determinants). Should a slot turn
+// out to need them (S_act too ill-conditioned, or a block that may be rank deficient), the launch is
+// repeated with them, and the pool's next kPairHold launches start with them.
+constexpr int kPairHold = 64;
+void evaluate_now(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
+                  const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true) {
+    // a repeated Davidson solve would start from what the first one left
+    const bool strings_only = forward && p->pair_hold == 0 && p->eigensolver != VBE_EIGENSOLVER_DAVIDSON;
+    if (forward && p->pair_hold > 0) --p->pair_hold;
+    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed, strings_only);
+    if (!forward || lane.pair_kernels) return;
+    check(hipEventSynchronize(lane.done), "hipEventSynchronize");
+    bool left = false;
+    for (size_t i = 0; i < in.size(); ++i) {
+        const int* f = lane.h_flags + FLAG_COUNT * i;
+        left = left || !f[xmvb_amd::FLAG_STRINGS] || f[xmvb_amd::FLAG_NEAR];
+    }
+    if (!left) return;
+    p->pair_hold = kPairHold;
+    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed);
+}
+
 Lane& acquire_lane(vbe_pool* p) {
     for (int k = 0; k < kLanes; ++k) {
         Lane& l = p->lanes[(p->last_lane + 1 + k) % kLanes];
@@ -838,7 +947,7 @@ double eval_problem(vbe_problem* prob, const double* d_C, const uint8_t* d_suppo
     lane.busy = true;
     try {
         // a single problem's launch shape is the pinned one (the same bits as in any pinned batch)
-        enqueue(p, lane, in, want_grad, forward, nullptr, true);
+        evaluate_now(p, lane, in, want_grad, forward, nullptr, true);
     } catch (...) {
         lane.busy = false;
         throw;
@@ -866,7 +975,7 @@ void optimize_slots(vbe_pool* p, vbe_problem* prob, const std::vector<int>& slot
         lane.busy = true;
         try {
             // pinned: each slot follows the iterates it would follow alone, whatever the batch
-            enqueue(p, lane, in, with_grad, true, nullptr, true, false);
+            evaluate_now(p, lane, in, with_grad, true, nullptr, true, false);
         } catch (...) {
             lane.busy = false;
             throw;
@@ -935,12 +1044,14 @@ int eval_device_in_scratch(vbe_context* ctx, vbe_problem* prob, const double* d_
         const Slot& s = p->slots[0];
         if (!s.loaded) throw StatusError(VBE_ERR_ARGUMENT, "problem not loaded");
         SlotDesc ws = s.desc;
-        const size_t need = carve_workspace(p, s.n_bf, s.n_aux, nullptr, ws);
+        // without the string form where its arrays do not fit
+        const bool strings = carve_workspace(p, s.n_bf, s.n_aux, nullptr, ws) <= scratch_bytes;
+        const size_t need = carve_workspace(p, s.n_bf, s.n_aux, nullptr, ws, strings);
         if (need > scratch_bytes)
             throw StatusError(VBE_ERR_MEMORY, "evaluation workspace of " + std::to_string(need) +
                                                   " bytes exceeds the static scratch maximum of " +
                                                   std::to_string(scratch_bytes) + " bytes");
-        carve_workspace(p, s.n_bf, s.n_aux, scratch, ws);
+        carve_workspace(p, s.n_bf, s.n_aux, scratch, ws, strings);
         p->eigensolver = flags.eigensolver;
         check(hipSetDevice(ctx->device), "hipSetDevice");
         Lane& lane = p->lanes[0];
@@ -949,7 +1060,7 @@ int eval_device_in_scratch(vbe_context* ctx, vbe_problem* prob, const double* d_
         prob->forward_valid = false;
         lane.busy = true;
         try {
-            enqueue(p, lane, in, flags.want_gradient != 0, true, &ws);
+            evaluate_now(p, lane, in, flags.want_gradient != 0, true, &ws);
         } catch (...) {
             lane.busy = false;
             throw;
@@ -1272,7 +1383,7 @@ int vbe_pool_eval_device(vbe_pool* pool, int32_t count, const int32_t* slots, co
         }
         lane.busy = true;
         try {
-            enqueue(pool, lane, in, want_gradient != 0, true);
+            evaluate_now(pool, lane, in, want_gradient != 0, true);
         } catch (...) {
             lane.busy = false;
             throw;

@@ -540,6 +540,7 @@ __global__ void __launch_bounds__(512) k_pairs(const SlotDesc* __restrict__ slot
     constexpr int MB = GroupShape<GROUP>::MB;
     constexpr int GPW = 64 / GROUP;  // groups per wavefront
     const SlotDesc& sd = slots[blockIdx.z];
+    if (Backward && string_slot(sd)) return;
     const auto G_glob = to_global(sd.G);
     const int n = topo.n, ng = topo.ng, n_det = topo.n_det;
     const int np = n * (n + 1) / 2;
@@ -807,6 +808,7 @@ __global__ void __launch_bounds__(512) k_pairs(const SlotDesc* __restrict__ slot
 __global__ void k_reduce_partials(const SlotDesc* __restrict__ slots, int n_blocks, int len, int list_begin,
                                   int list_rows, int list_per_row) {
     const SlotDesc& sd = slots[blockIdx.z];
+    if (string_slot(sd)) return;
     const auto partials = to_global(sd.partials);
     const auto out = to_global(sd.dsum);
     const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -830,6 +832,7 @@ constexpr int kReduceRowsFew = 64;
 __global__ void __launch_bounds__(256) k_reduce_partials_few(const SlotDesc* __restrict__ slots, int n_blocks, int len,
                                                              int list_begin, int list_rows, int list_per_row) {
     const SlotDesc& sd = slots[blockIdx.z];
+    if (string_slot(sd)) return;
     const auto partials = to_global(sd.partials);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= len) return;
@@ -860,7 +863,10 @@ struct CompactView {
     __device__ CompactView(const SlotDesc& sd, const TopoDesc& topo, int listed) {
         flag = Deferred ? sd.defer_flag : sd.singular_flag;
         out = Deferred ? sd.defer : sd.singular;
-        entries = Deferred ? topo.n_lane_pairs
+        // the string form defers pairs only where some block may be rank deficient
+        const bool none = Deferred && string_slot(sd) && !to_global(sd.flags)[FLAG_NEAR];
+        entries = none ? 0
+                  : Deferred ? topo.n_lane_pairs
                   : listed ? (long long)to_global(sd.flags)[FLAG_DEFERRED]
                            : (long long)topo.n_det * (topo.n_det + 1) / 2;
     }
@@ -2226,6 +2232,7 @@ hipError_t configure_kernels(int n, int ng, int n_str, int mmax) {
     if ((e = configure_pairs_lane()) != hipSuccess) return e;
     if ((e = configure_ri_tiled()) != hipSuccess) return e;
     if ((e = configure_pairs_singular()) != hipSuccess) return e;
+    if ((e = configure_strings()) != hipSuccess) return e;
     return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gep_lowest<true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGepLdsLimit);
 }
@@ -2280,11 +2287,14 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
     if (fork) {
         (void)hipEventRecord(side->fork, st);
         (void)hipStreamWaitEvent(side->st, side->fork, 0);
-        hipLaunchKernelGGL(k_active_matrices, dim3(1, 1, z), dim3(256), 0, side->st, slots, n);
-        (void)hipEventRecord(side->join, side->st);
-    } else {
-        hipLaunchKernelGGL(k_active_matrices, dim3(1, 1, z), dim3(256), 0, st, slots, n);
     }
+    const hipStream_t active = fork ? side->st : st;
+    hipLaunchKernelGGL(k_active_matrices, dim3(1, 1, z), dim3(256), 0, active, slots, n);
+    if (shape.strings) {
+        launch_string_frame(active, slots, z, topo);
+        launch_string_minors(active, slots, z, topo);
+    }
+    if (fork) (void)hipEventRecord(side->join, side->st);
     mark(EV_PREP);
     if (shape.any_tiled)
         launch_ri_one_index_tiled(st, slots, count, n, shape.max_n_bf_tiled, shape.max_n_aux, shape.b32c);
@@ -2325,20 +2335,27 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
         hipLaunchKernelGGL(k_ri_pair_gram_tiled, dim3(1, 1, z), dim3(256), 0, st, slots, np);
     if (fork) (void)hipStreamWaitEvent(st, side->join, 0);
     mark(EV_TRANSFORM);
-    if (shape.lane_fwd) {
+    const long long all_pairs = (long long)topo.n_det * (topo.n_det + 1) / 2;
+    if (shape.strings) {
+        launch_string_integrals(st, slots, z, topo);
+        launch_string_forward(st, slots, z, topo);
+    }
+    if (!shape.pair_kernels) {
+        mark(EV_PAIR_FWD_MAIN);
+    } else if (shape.lane_fwd) {
+        if (shape.strings) launch_string_defer(st, slots, z, topo);
         launch_pairs_lane(st, 0, shape.lane_blocks_fwd, slots, count, topo, shape.n_alpha, shape.n_beta,
                           shape.lane_cond_limit);
         mark(EV_PAIR_FWD_MAIN);
-        const long long all_pairs = (long long)topo.n_det * (topo.n_det + 1) / 2;
         compact_pairs<true>(st, slots, z, topo, 1, topo.n_lane_pairs);
         launch_pairs_group(st, false, true, shape.list_blocks, 0, slots, count, topo, shape.mmax);
         compact_pairs<false>(st, slots, z, topo, 1, all_pairs);
     } else {
         launch_pairs_group(st, false, false, shape.pair_blocks_fwd, 0, slots, count, topo, shape.mmax);
         mark(EV_PAIR_FWD_MAIN);
-        compact_pairs<false>(st, slots, z, topo, 0, (long long)topo.n_det * (topo.n_det + 1) / 2);
+        compact_pairs<false>(st, slots, z, topo, 0, all_pairs);
     }
-    launch_pairs_singular(st, false, 0, slots, count, topo);
+    if (shape.pair_kernels) launch_pairs_singular(st, false, 0, slots, count, topo);
     mark(EV_PAIR_FWD);
     const long long a = (long long)topo.n_det * topo.n_str, b = (long long)topo.n_str * topo.n_str;
     hipLaunchKernelGGL(k_structure_right, dim3((unsigned)((a + 255) / 256), 1, z), dim3(256), 0, st, slots, topo);
@@ -2386,49 +2403,54 @@ void launch_backward(hipStream_t st, const SlotDesc* slots, int count, const Top
         if (ev) (void)hipEventRecord(ev[k], st);
     };
     mark(EV_BWD_BEGIN);
-    // The pair-adjoint kernels write disjoint columns (field: ds/dh; adjoint: dg) or disjoint rows
-    // (deferred list, singular pairs) of the partial rows, so for few problems the adjoint kernel and
-    // the singular-pair kernel run on the side stream beside the field and deferred-list kernels.
-    const bool fork = side && count <= kForkMaxProblems && shape.lane_bwd;
-    hipStream_t st2 = st;
-    if (fork) {
-        (void)hipEventRecord(side->fork, st);
-        (void)hipStreamWaitEvent(side->st, side->fork, 0);
-        st2 = side->st;
-    }
-    int part_rows = shape.pair_blocks_bwd, list_begin = 0, list_rows = 0, list_per_row = 1;
-    if (shape.lane_bwd) {
-        launch_pairs_lane(st, 1, shape.lane_blocks_bwd, slots, count, topo, shape.n_alpha, shape.n_beta,
-                          shape.lane_cond_limit);
-        mark(EV_BWD_FIELD);
-        launch_pairs_lane(st2, 2, shape.lane_blocks_bwd, slots, count, topo, shape.n_alpha, shape.n_beta,
-                          shape.lane_cond_limit);
-        if (!fork) mark(EV_BWD_ADJOINT);
-        list_per_row = launch_pairs_group(st, true, true, shape.list_blocks, shape.lane_blocks_bwd, slots, count, topo,
-                                          shape.mmax);
-        list_begin = shape.lane_blocks_bwd;
-        list_rows = shape.list_blocks;
-        part_rows = shape.lane_blocks_bwd + shape.list_blocks;
+    if (shape.strings) launch_string_backward(st, slots, z, topo);
+    if (!shape.pair_kernels) {
+        for (const int k : {EV_BWD_FIELD, EV_BWD_ADJOINT, EV_BWD_KERNEL}) mark(k);
     } else {
-        launch_pairs_group(st, true, false, shape.pair_blocks_bwd, 0, slots, count, topo, shape.mmax);
-        mark(EV_BWD_FIELD);
-        mark(EV_BWD_ADJOINT);
+        // The pair-adjoint kernels write disjoint columns (field: ds/dh; adjoint: dg) or disjoint rows
+        // (deferred list, singular pairs) of the partial rows, so for few problems the adjoint kernel and
+        // the singular-pair kernel run on the side stream beside the field and deferred-list kernels.
+        const bool fork = side && count <= kForkMaxProblems && shape.lane_bwd && !shape.strings;
+        hipStream_t st2 = st;
+        if (fork) {
+            (void)hipEventRecord(side->fork, st);
+            (void)hipStreamWaitEvent(side->st, side->fork, 0);
+            st2 = side->st;
+        }
+        int part_rows = shape.pair_blocks_bwd, list_begin = 0, list_rows = 0, list_per_row = 1;
+        if (shape.lane_bwd) {
+            launch_pairs_lane(st, 1, shape.lane_blocks_bwd, slots, count, topo, shape.n_alpha, shape.n_beta,
+                              shape.lane_cond_limit);
+            mark(EV_BWD_FIELD);
+            launch_pairs_lane(st2, 2, shape.lane_blocks_bwd, slots, count, topo, shape.n_alpha, shape.n_beta,
+                              shape.lane_cond_limit);
+            if (!fork) mark(EV_BWD_ADJOINT);
+            list_per_row = launch_pairs_group(st, true, true, shape.list_blocks, shape.lane_blocks_bwd, slots, count, topo,
+                                              shape.mmax);
+            list_begin = shape.lane_blocks_bwd;
+            list_rows = shape.list_blocks;
+            part_rows = shape.lane_blocks_bwd + shape.list_blocks;
+        } else {
+            launch_pairs_group(st, true, false, shape.pair_blocks_bwd, 0, slots, count, topo, shape.mmax);
+            mark(EV_BWD_FIELD);
+            mark(EV_BWD_ADJOINT);
+        }
+        launch_pairs_singular(st2, true, part_rows, slots, count, topo);
+        part_rows += kSingularBlocks;
+        if (fork) {
+            (void)hipEventRecord(side->join, side->st);
+            (void)hipStreamWaitEvent(st, side->join, 0);
+            mark(EV_BWD_ADJOINT);  // field and deferred list done on the main stream, adjoint joined
+        }
+        mark(EV_BWD_KERNEL);
+        const int len = ng + 2 * n * n;
+        if (part_rows <= kReduceRowsFew)
+            hipLaunchKernelGGL(k_reduce_partials_few, dim3((len + 255) / 256, 1, z), dim3(256), 0, st, slots, part_rows,
+                               len, list_begin, list_rows, list_per_row);
+        else
+            hipLaunchKernelGGL(k_reduce_partials, dim3((len + 3) / 4, 1, z), dim3(256), 0, st, slots, part_rows, len,
+                               list_begin, list_rows, list_per_row);
     }
-    launch_pairs_singular(st2, true, part_rows, slots, count, topo);
-    part_rows += kSingularBlocks;
-    if (fork) {
-        (void)hipEventRecord(side->join, side->st);
-        (void)hipStreamWaitEvent(st, side->join, 0);
-        mark(EV_BWD_ADJOINT);  // field and deferred list done on the main stream, adjoint joined
-    }
-    mark(EV_BWD_KERNEL);
-    const int len = ng + 2 * n * n;
-    if (part_rows <= kReduceRowsFew)
-        hipLaunchKernelGGL(k_reduce_partials_few, dim3((len + 255) / 256, 1, z), dim3(256), 0, st, slots, part_rows,
-                           len, list_begin, list_rows, list_per_row);
-    else
-        hipLaunchKernelGGL(k_reduce_partials, dim3((len + 3) / 4, 1, z), dim3(256), 0, st, slots, part_rows, len,
-                           list_begin, list_rows, list_per_row);
     mark(EV_PAIR_BWD);
     hipLaunchKernelGGL(k_ri_pair_adjoint, dim3((shape.max_n_aux + 255) / 256, (np + 7) / 8, z), dim3(256), 0, st, slots,
                        np);

@@ -11,6 +11,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "strings.hpp"
+
 namespace xmvb_amd {
 
 // Largest active space handled by the LDS-resident determinant-pair kernels.
@@ -28,6 +30,8 @@ enum DeviceFlag : int {
     FLAG_METRIC = 3,          // structure metric not positive definite
     FLAG_DEFERRED = 4,        // pairs left by the lane kernel for the lane-group kernel (SlotDesc::defer)
     FLAG_EIGEN = 5,           // Davidson stopped without meeting its tolerances (1 + reason)
+    FLAG_STRINGS = 6,         // the slot takes the string form instead of the pair kernels
+    FLAG_NEAR = 7,            // string form: some block may be rank deficient (StringWork::neara, nearb)
     FLAG_COUNT = 8
 };
 
@@ -64,6 +68,7 @@ struct SlotDesc {
     uint8_t* singular_flag;  // per lane-group entry: rank deficient (listed into singular in order)
     int* chunk_count;        // list compaction: entries listed per chunk of kCompactChunk, then offsets
     double* state_energy;    // eigenvalue of each selected state (kMaxStates; n_states > 1 only)
+    StringWork sw;           // arrays of the string form (null without one)
     int seeded;     // coef holds this slot's previous structure eigenvector (Davidson start)
 };
 
@@ -95,6 +100,7 @@ struct TopoDesc {
     int n_states;
     int state_idx[kMaxStates];
     double state_w[kMaxStates];
+    StringTopo str;
 };
 
 struct LaunchShape {
@@ -110,6 +116,8 @@ struct LaunchShape {
     bool b32c;                             // RI factors stored as compensated FP32 (FP32 + 8-bit correction)
     bool any_tiled, any_flat;              // slots of the launch with the aux-tiled / the flat layout
     int max_n_bf_tiled;                    // largest n_bf among the slots with the aux-tiled layout
+    bool strings;                          // slots may take the string form (their FLAG_STRINGS decides)
+    bool pair_kernels;                     // launch the pair kernels too, for slots or pairs the string form leaves
     bool davidson;                         // structure eigenproblem by Davidson instead of dense
     // Pinned launch shape: every choice that changes a slot's summation order (blocks per slot of the
     // backward pair kernels, the few-problem or batched form of the Gram product, gradient tail and

@@ -477,6 +477,7 @@ template <int M0, int M1>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lane_fwd_waves(M0))))
     k_pairs_lane_fwd(const SlotDesc* __restrict__ slots, TopoDesc topo, int swap_spins, double cond_limit) {
     const SlotDesc& sd = slots[blockIdx.z];
+    if (string_slot(sd)) return;
     const int n = topo.n, n_det = topo.n_det;
     const int np = n * (n + 1) / 2;
     extern __shared__ double lds[];
@@ -569,6 +570,7 @@ template <int M0, int M1>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lane_field_waves(M0))))
     k_pairs_lane_bwd_f(const SlotDesc* __restrict__ slots, TopoDesc topo, int swap_spins, double cond_limit) {
     const SlotDesc& sd = slots[blockIdx.z];
+    if (string_slot(sd)) return;
     const int n = topo.n, ng = topo.ng;
     const int np = n * (n + 1) / 2;
     extern __shared__ double lds[];
@@ -683,6 +685,7 @@ __global__ void __launch_bounds__(256)
     k_pairs_lane_bwd_g(const SlotDesc* __restrict__ slots, TopoDesc topo, int swap_spins, double cond_limit,
                        LaneBwdLayout lay) {
     const SlotDesc& sd = slots[blockIdx.z];
+    if (string_slot(sd)) return;
     const int n = topo.n, ng = topo.ng;
     const int np = n * (n + 1) / 2;
     extern __shared__ double lds[];

@@ -378,6 +378,7 @@ template <bool Backward, bool FullDg>
 __global__ void __launch_bounds__(256) k_pairs_singular(const SlotDesc* __restrict__ slots, TopoDesc topo,
                                                         int part_offset) {
     const SlotDesc& sd = slots[blockIdx.z];
+    if (Backward && string_slot(sd)) return;
     const int n = topo.n, ng = topo.ng, n_det = topo.n_det;
     const int np = n * (n + 1) / 2;
     const int count = to_global(sd.flags)[FLAG_SINGULAR_PAIRS];

@@ -1,0 +1,149 @@
+// Evaluation over the strings of the active space ("string form"), see strings.hip.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+namespace xmvb_amd {
+
+// All strings of m electrons in n orbitals, in ascending mask order, with their single replacements:
+// e1[x * J + j], j < noff: l -> q with q unoccupied, then the m occupied orbitals (q == l). An entry
+// packs the rank of the resulting string (bits 0-15), q n + l (16-23) and the parity (31).
+struct StringSpace {
+    int m, N, noff, J;
+    const uint32_t* mask;
+    const uint32_t* e1;
+};
+
+// One determinant reached from a string row: determinant, and packed (rank or orbital pair, parity).
+struct StringLink {
+    uint32_t det;
+    uint32_t to;  // bits 0-15: rank of the replaced string, or q n + l (n^2: no replacement); 31: parity
+};
+
+// A determinant (negative: padding) with its string ranks and its spin-flip partner (itself without one).
+struct StringDet {
+    int det, a, b, flip;
+};
+
+// Determinant pairs {order[begin..end), det}, those with order_couple(position) <= couple.
+struct StringPairItem {
+    int det, begin, end, couple;
+};
+
+// Couple of a position of the order: blocks of sixteen hold one determinant of each of eight couples, then
+// their partners, so that either half runs along consecutive strings.
+__host__ __device__ inline int order_couple(int position, bool flip) {
+    return flip ? 8 * (position >> 4) + (position & 7) : position;
+}
+
+// Topology tables of the string form (device pointers).
+struct StringTopo {
+    int enabled;  // 0: this topology takes the pair kernels
+    int sym;      // +-1: exchanging the spins multiplies every determinant coefficient by it; 0: no such sign
+    StringSpace a, b;
+    const uint16_t* rank;              // mask -> rank among the masks of the same electron count
+    const int *arank, *brank;          // determinant -> string ranks
+    const int *aoff, *adet;            // alpha string -> determinants
+    const int *boff, *bdet;            // beta string -> determinants
+    const int* soff;                   // alpha string -> determinants one alpha replacement away
+    const StringLink* slink;
+    const int* goff;                   // (q, l) -> determinants whose alpha string allows l -> q
+    const StringLink* glink;
+    int gchunks;                       // chunks of 64 links of the longest (q, l) list
+    // determinant pairs: the determinants in order (order_couple) and the wavefront items of k_string_pairs
+    const StringDet* order;
+    const StringPairItem* pitem;
+    int npitem;
+    // alpha strings for the same, as offsets x * J + j per (q, l): [ak][n^2], ~0 past the end
+    const uint32_t* alist;
+    int ak;
+    // strings of one beta electron fewer, [nw][16]: rank of the string with orbital q added (bits 0-11; N
+    // where q is occupied or past n) and the parity of q's place (15)
+    const uint16_t* wtab;
+    // double replacements l < l2 -> q < q2 of every string (q, q2 may be l, l2), [N][pairs l l2][nq]: rank
+    // (0-11), compound index of (q, q2) (12-18), parity (31)
+    const uint32_t *e2a, *e2b;
+    // (l, l2) -> determinants whose beta (alpha) string holds both, and the place of l l2 among its pairs
+    const int *w2off_b, *w2off_a;
+    const StringLink *w2link_b, *w2link_a;
+    int nw, nq_a, nq_b, wchunks;
+};
+
+// Host image of the tables, built once per pool.
+struct StringTables {
+    bool enabled = false;
+    int sym = 0, n = 0;
+    struct Space {
+        int m = 0, N = 0, noff = 0, J = 0;
+        std::vector<uint32_t> mask, e1;
+    } a, b;
+    std::vector<uint16_t> rank;
+    std::vector<int> arank, brank, aoff, adet, boff, bdet, soff, goff;
+    std::vector<StringLink> slink, glink;
+    std::vector<uint32_t> alist, e2a, e2b;
+    std::vector<uint16_t> wtab;
+    std::vector<StringDet> order;
+    std::vector<StringPairItem> pitem;
+    std::vector<int> w2off_a, w2off_b;
+    std::vector<StringLink> w2link_a, w2link_b;
+    int gchunks = 0, ak = 0, nw = 0, nq_a = 0, nq_b = 0, wchunks = 0;
+};
+
+StringTables build_string_tables(int n, int n_alpha, int n_beta, int n_det, const uint64_t* amask, const int* det_a,
+                                 const uint64_t* bmask, const int* det_b, const long long* off, const int* ts,
+                                 const double* tc, const std::vector<int>& flip);
+
+// Arrays of one slot. The determinant matrices are dead once the structure matrices are formed, so
+// f and sigma (with C M before it) take their place.
+struct StringWork {
+    double *Sinv, *ht;   // S_act^-1, S_act^-1 h_act (n x n, row-major)
+    double *U, *gt;      // S_act^-1 on one, on both sides of the packed kernel: [q n + l][pair], [q n + l][q2 n + l2]
+    double *Ma, *Mb;     // minors of S_act over all string pairs
+    double *Ja, *Jb;     // sum over the occupied l2 of gt[q n + l][l2 l2], per string
+    double *Ha, *Hb;     // same-spin Hamiltonian in the dual frame, [x][a]
+    unsigned char *neara, *nearb;  // string pairs whose overlap block may be rank deficient
+    double *Ka, *Kb;     // same-spin Hamiltonian between strings; during the forward, over gpart and on
+    double *gpart, *wpart, *zpart;
+    double *gs, *hb, *V, *W2, *Zt;
+    double *Fa, *Fb;     // ht + Coulomb - exchange of each string, [x][ql]
+};
+
+// Where the string form is the faster one (both measured in one build, in us, string form / pair kernels):
+// one problem of 70, 126, 252, 462 determinants 372/345, 528/460, 515/506, 2326/2718; 32 problems
+// 402/389, 651/749, 747/1469, 4446/12988. So always from kStringDets on, and from kStringDetsBatched for
+// launches of at least kStringBatch problems (never for pinned shapes, whose form may not depend on the batch).
+constexpr int kStringDets = 200, kStringDetsBatched = 100, kStringBatch = 16;
+constexpr int kStringRowsZ = 8;         // rows of f and sigma per workgroup of the response sum
+constexpr int kStringPairSegment = 128; // determinants per wavefront of k_string_pairs (512 in large spaces)
+// A block whose smallest singular value is provably above this is regular under the complete-pivoting rank
+// rule: its pivots are at least sigma_min / m and at most 16 max|X| <= 16, a ratio above 7e-12 for m <= 8
+// against the rule's 1e-12, and no singular value is below the rule's absolute 1e-12.
+constexpr double kStringRegularSigma = 1.0e-9;
+// Largest |S_act^-1| element (orbitals of unit norm) for which a slot takes the string form.
+constexpr double kStringInverseLimit = 16.0;
+
+struct SlotDesc;
+struct TopoDesc;
+
+// layout of a slot's StringWork in one block of doubles (base null: only counted); returns their number
+std::size_t string_work_carve(const TopoDesc& topo, double* base, StringWork& w);
+
+// S_act^-1 and the route of each slot (FLAG_STRINGS); after the active matrices
+void launch_string_frame(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+// minors of S_act and the blocks that may be rank deficient
+void launch_string_minors(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+// transformed integrals and the same-spin Hamiltonian
+void launch_string_integrals(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+// determinant matrices (SlotDesc::Hdet, Sdet)
+void launch_string_forward(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+// flags of the pairs with a block that may be rank deficient, left to the lane-group kernel
+void launch_string_defer(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+// adjoints of the packed kernel, S_act and h_act into SlotDesc::dsum
+void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+hipError_t configure_strings();
+
+}  // namespace xmvb_amd
