@@ -21,5 +21,6 @@ __device__ __forceinline__ gptr<T> to_global(T* p) {
 // whose assignment does not bind to an address-space-qualified operand)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));  // at any double
 
 }  // namespace xmvb_amd

@@ -1042,20 +1042,15 @@ __global__ void k_structure_left(const SlotDesc* __restrict__ slots, TopoDesc to
 
 
 // ---------------------------------------------------------------------------------------------
-// generalised eigenproblem H c = E S c, lowest root, one workgroup.
-// Cholesky S = L L^T, explicit L^{-1}, M = L^{-1} H L^{-T} by two triangular products,
-// Householder tridiagonalisation, multisection on Sturm counts for the lowest eigenvalue, inverse
-// iteration on the tridiagonal, back-transformation, c = L^{-T} z so that c^T S c = 1.
-// Storage: gep_work_doubles(n) = 3*n*n + 9*n doubles, in LDS when it fits (InLds) else in the
-// global workspace. A single wavefront is used for small n so that the block barriers are free.
+// generalised eigenproblem H c = E S c beyond one wavefront (n_str > 64): Cholesky S = L L^T, explicit
+// L^{-1}, A = L^{-1} H L^{-T} by two triangular products, its lowest eigenpair by Lanczos
+// (gep_large.hip, to 1024 structures), c = L^{-T} z so that c^T S c = 1. Selected states and larger spaces take
+// the whole reduction: Householder tridiagonalisation, multisection on Sturm counts, inverse
+// iteration on the tridiagonal, back-transformation.
+// Workspace gep_work_doubles(n): L, A, L^{-1} column-major (n x n each), 9 n vectors, then two more n x n.
 // ---------------------------------------------------------------------------------------------
-// Front half of the eigensolver for n_str whose matrices live in global memory, over many
-// workgroups: k_gep_chol (one workgroup per problem: symmetrised S and H, Cholesky S = L L^T in
-// place), k_gep_linv (L^-1 by independent columns, one wavefront per column: X1 holds it row-major and
-// V column-major), k_gep_hlt (U = H L^-T into X2) and k_gep_lul (A = L^-1 U into M), after which
-// k_gep_lowest<false, 3> continues from the symmetrisation of A (launches of few problems replace
-// the Cholesky and the Householder stage by the per-step kernels further down). Workspace layout
-// as in k_gep_lowest (Lm, M, V, 9 n vectors) followed by X1, X2.
+// Front half over many workgroups: the Cholesky (in LDS, blocked over launches, or k_gep_chol on one
+// workgroup per problem), the columns of L^{-1}, k_gep_hlt (U = H L^{-T}) and k_gep_lul (A = L^{-1} U).
 __device__ __forceinline__ size_t gep_core_dev(int n) { return 3 * (size_t)n * n + 9 * (size_t)n; }
 
 __global__ void __launch_bounds__(1024) k_gep_chol(const SlotDesc* __restrict__ slots, TopoDesc topo) {
@@ -1089,52 +1084,15 @@ __global__ void __launch_bounds__(1024) k_gep_chol(const SlotDesc* __restrict__ 
     }
 }
 
-// X = L^-1 by columns, one wavefront per column j: X[i][j] = (delta_ij - sum_{k=j}^{i-1} L[i][k]
-// X[k][j]) / L[i][i] for i = j..n-1 in order, each sum split over the 64 lanes, the column kept in
-// LDS as it grows. grid (ceil(n/4), 1, slots), 256 threads, dynamic LDS 4 n doubles
-// (n <= kLinvWaveMaxN; larger n take k_gep_linv_lane).
-constexpr int kLinvWaveMaxN = 2048;
-
-__global__ void __launch_bounds__(256) k_gep_linv(const SlotDesc* __restrict__ slots, int n) {
-    const SlotDesc& sd = slots[blockIdx.z];
-    const auto L = to_global(sd.gep);
-    const auto V = to_global(sd.gep) + 2 * (size_t)n * n;
-    const auto X1 = to_global(sd.gep) + gep_core_dev(n);
-    extern __shared__ double xs[];  // four columns of n
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int j = blockIdx.x * 4 + wave;
-    if (j >= n) return;  // wave-uniform; the kernel has no block barrier
-    double* x = xs + (size_t)wave * n;
-    for (int i = lane; i < j; i += 64) {
-        X1[j + (size_t)n * i] = 0.0;
-        V[i + (size_t)n * j] = 0.0;
-    }
-    for (int i = j; i < n; ++i) {
-        double s = 0.0;
-        for (int k = j + lane; k < i; k += 64) s += L[i + (size_t)n * k] * x[k];
-        s = wave_sum(s);
-        const double xi = ((i == j) ? 1.0 - s : -s) / L[i + (size_t)n * i];
-        if (lane == 0) {
-            x[i] = xi;
-            X1[j + (size_t)n * i] = xi;  // row-major: X1[j + n i] = X[i][j]
-            V[i + (size_t)n * j] = xi;   // column-major
-        }
-        wave_sync();  // x[i] is visible to every lane before row i + 1
-    }
-}
-
-// The same with one lane per column (no LDS; for n above kLinvWaveMaxN).
+// V = L^-1 (column-major) with one lane per column, for spaces beyond launch_gep_linv_cols.
 __global__ void __launch_bounds__(64) k_gep_linv_lane(const SlotDesc* __restrict__ slots, int n) {
     const SlotDesc& sd = slots[blockIdx.z];
     const auto L = to_global(sd.gep);
     const auto V = to_global(sd.gep) + 2 * (size_t)n * n;
-    const auto X1 = to_global(sd.gep) + gep_core_dev(n);
+    const auto X1 = to_global(sd.gep) + gep_core_dev(n);  // row-major copy: the lanes' own sums read it
     const int j = blockIdx.x * 64 + threadIdx.x;
     if (j >= n) return;
-    for (int i = 0; i < j; ++i) {
-        X1[j + (size_t)n * i] = 0.0;
-        V[i + (size_t)n * j] = 0.0;
-    }
+    for (int i = 0; i < j; ++i) V[i + (size_t)n * j] = 0.0;
     for (int i = j; i < n; ++i) {
         double s0 = (i == j) ? 1.0 : 0.0, s1 = 0.0;
         int k = j;
@@ -1153,44 +1111,46 @@ __global__ void __launch_bounds__(64) k_gep_linv_lane(const SlotDesc* __restrict
 __global__ void __launch_bounds__(256) k_gep_hlt(const SlotDesc* __restrict__ slots, int n) {
     const SlotDesc& sd = slots[blockIdx.z];
     const auto H = to_global(sd.gep) + (size_t)n * n;  // M holds the symmetrised H
-    const auto X1 = to_global(sd.gep) + gep_core_dev(n);
+    const auto V = to_global(static_cast<const double*>(sd.gep)) + 2 * (size_t)n * n;
     const auto X2 = to_global(sd.gep) + gep_core_dev(n) + (size_t)n * n;
     const int i = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y;
     if (i >= n) return;
     double s0 = 0.0, s1 = 0.0;
     int k = 0;
+#pragma unroll 4
     for (; k + 1 <= j; k += 2) {
-        s0 += H[i + (size_t)n * k] * X1[k + (size_t)n * j];
-        s1 += H[i + (size_t)n * (k + 1)] * X1[k + 1 + (size_t)n * j];
+        s0 += H[i + (size_t)n * k] * V[j + (size_t)n * k];
+        s1 += H[i + (size_t)n * (k + 1)] * V[j + (size_t)n * (k + 1)];
     }
-    for (; k <= j; ++k) s0 += H[i + (size_t)n * k] * X1[k + (size_t)n * j];
+    for (; k <= j; ++k) s0 += H[i + (size_t)n * k] * V[j + (size_t)n * k];
     X2[i + (size_t)n * j] = s0 + s1;
 }
 
-// A = L^-1 U: A[i][j] = sum_{k<=i} X[i][k] U[k][j] into M (thread = row i, grid y = column j)
+// A = L^-1 U: A[i][j] = sum_{k<=i} X[i][k] U[k][j] into M (thread = row i, grid y = column j), the lower
+// triangle mirrored
 __global__ void __launch_bounds__(256) k_gep_lul(const SlotDesc* __restrict__ slots, int n) {
     const SlotDesc& sd = slots[blockIdx.z];
     const auto A = to_global(sd.gep) + (size_t)n * n;
     const auto V = to_global(sd.gep) + 2 * (size_t)n * n;
     const auto X2 = to_global(sd.gep) + gep_core_dev(n) + (size_t)n * n;
     const int i = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y;
-    if (i >= n) return;
+    if (i >= n || i < j) return;
     double s0 = 0.0, s1 = 0.0;
     int k = 0;
+#pragma unroll 4
     for (; k + 1 <= i; k += 2) {
         s0 += V[i + (size_t)n * k] * X2[k + (size_t)n * j];
         s1 += V[i + (size_t)n * (k + 1)] * X2[k + 1 + (size_t)n * j];
     }
     for (; k <= i; ++k) s0 += V[i + (size_t)n * k] * X2[k + (size_t)n * j];
     A[i + (size_t)n * j] = s0 + s1;
+    if (i != j) A[j + (size_t)n * i] = s0 + s1;
 }
 
-// Blocked Cholesky of the large-n path for launches of few problems: k_gep_load symmetrises S
-// and H into the workspace (many blocks); then per panel of kCholPanel columns j0.. j0+jb-1:
-// k_chol_diag factors the diagonal tile in LDS (one block; a pivot a <= 0 sets the metric flag
-// and the solve goes on with values the host discards), k_chol_trsm solves the rows below it
-// against the tile (one thread per row), k_chol_syrk subtracts the panel's product from the
-// trailing lower triangle (16 x 16 tiles). About 3 n / kCholPanel launches instead of 2 n.
+// k_gep_load symmetrises S and H into the workspace (many blocks). Blocked Cholesky of the large-n path
+// for launches of few problems: per panel of kCholPanel columns j0.. j0+jb-1:
+// k_chol_panel (gep_large.hip) factors the diagonal tile and solves the rows below it, k_chol_syrk
+// subtracts the panel's product from the trailing lower triangle (16 x 16 tiles). About 2 n / kCholPanel launches instead of 2 n.
 __global__ void __launch_bounds__(256) k_gep_load(const SlotDesc* __restrict__ slots, int n) {
     const SlotDesc& sd = slots[blockIdx.z];
     const auto Lm = to_global(sd.gep);
@@ -1202,70 +1162,20 @@ __global__ void __launch_bounds__(256) k_gep_load(const SlotDesc* __restrict__ s
     M[idx] = 0.5 * (sd.Hs[i + (size_t)n * j] + to_global(sd.Hs)[j + (size_t)n * i]);
 }
 
-constexpr int kCholPanel = 32;
-
-__global__ void __launch_bounds__(256) k_chol_diag(const SlotDesc* __restrict__ slots, int n, int j0, int jb) {
-    const SlotDesc& sd = slots[blockIdx.z];
-    const auto L = to_global(sd.gep);
-    __shared__ double t[kCholPanel][kCholPanel + 1];  // t[i][j], lower triangle
-    for (int idx = threadIdx.x; idx < jb * jb; idx += blockDim.x) {
-        const int i = idx % jb, j = idx / jb;
-        t[i][j] = L[(size_t)(j0 + i) + (size_t)n * (j0 + j)];
-    }
-    __syncthreads();
-    for (int k = 0; k < jb; ++k) {
-        const double a = t[k][k];
-        if (!(a > 0.0) && threadIdx.x == 0) to_global(sd.flags)[FLAG_METRIC] = 1;
-        const double dk = sqrt(a), rdk = 1.0 / dk;
-        __syncthreads();  // every thread has read the pivot before it is replaced
-        for (int i = k + threadIdx.x; i < jb; i += blockDim.x) t[i][k] = (i == k) ? dk : t[i][k] * rdk;
-        __syncthreads();
-        const int m = jb - k - 1;
-        for (int idx = threadIdx.x; idx < m * m; idx += blockDim.x) {
-            const int i = k + 1 + idx % m, j = k + 1 + idx / m;
-            if (j <= i) t[i][j] -= t[i][k] * t[j][k];
-        }
-        __syncthreads();
-    }
-    for (int idx = threadIdx.x; idx < jb * jb; idx += blockDim.x) {
-        const int i = idx % jb, j = idx / jb;
-        if (j <= i) L[(size_t)(j0 + i) + (size_t)n * (j0 + j)] = t[i][j];
-    }
-}
-
-// rows i >= j0 + jb: L[i][j0..j0+jb) = A[i][j0..j0+jb) L_tile^-T (forward substitution per row)
-__global__ void __launch_bounds__(256) k_chol_trsm(const SlotDesc* __restrict__ slots, int n, int j0, int jb) {
-    const SlotDesc& sd = slots[blockIdx.z];
-    const auto L = to_global(sd.gep);
-    __shared__ double t[kCholPanel][kCholPanel + 1];
-    for (int idx = threadIdx.x; idx < jb * jb; idx += blockDim.x) {
-        const int i = idx % jb, j = idx / jb;
-        t[i][j] = j <= i ? L[(size_t)(j0 + i) + (size_t)n * (j0 + j)] : 0.0;
-    }
-    __syncthreads();
-    const int i = j0 + jb + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double x[kCholPanel];
-#pragma unroll
-    for (int j = 0; j < kCholPanel; ++j) {
-        if (j < jb) {
-            double v = L[(size_t)i + (size_t)n * (j0 + j)];
-#pragma unroll
-            for (int k = 0; k < j; ++k) v -= x[k] * t[j][k];
-            x[j] = v / t[j][j];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kCholPanel; ++j)
-        if (j < jb) L[(size_t)i + (size_t)n * (j0 + j)] = x[j];
-}
-
-// trailing update: A[i][j] -= sum_k L[i][j0+k] L[j][j0+k] for j0 + jb <= j <= i < n, 16 x 16 tiles
+// trailing update: A[i][j] -= sum_k L[i][j0+k] L[j][j0+k] for j0 + jb <= j <= i < n, 16 x 16 tiles; the first
+// workgroup also puts the panel's factored diagonal tile into L
 __global__ void __launch_bounds__(256) k_chol_syrk(const SlotDesc* __restrict__ slots, int n, int j0, int jb) {
     const int ti = blockIdx.x, tj = blockIdx.y;
     if (tj > ti) return;  // block-uniform: tiles above the diagonal
     const SlotDesc& sd = slots[blockIdx.z];
     const auto L = to_global(sd.gep);
+    if (ti == 0) {
+        const auto scratch = L + gep_core_dev(n);
+        for (int idx = threadIdx.x; idx < kCholPanel * kCholPanel; idx += 256) {
+            const int r = idx / kCholPanel, k = idx % kCholPanel;
+            if (k <= r) L[(size_t)(j0 + r) + (size_t)n * (j0 + k)] = scratch[idx];
+        }
+    }
     __shared__ double li[16][kCholPanel + 1], lj[16][kCholPanel + 1];
     const int r0 = j0 + jb + 16 * ti, c0 = j0 + jb + 16 * tj;
     for (int idx = threadIdx.x; idx < 16 * jb; idx += blockDim.x) {
@@ -1400,32 +1310,23 @@ __global__ void __launch_bounds__(256) k_hh_finish(const SlotDesc* __restrict__ 
     }
 }
 
-// Part 0: the whole solve (matrices in LDS). Large-n path (matrices in global memory, after the
-// multi-workgroup front half): Part 3 is the rest on one workgroup per problem (batched launches);
-// for launches of few problems, Part 1 is the symmetrisation and Part 2 the rest after the
+// After the multi-workgroup front half: Part 3 is the rest on one workgroup per problem (batched
+// launches); for launches of few problems, Part 1 is the symmetrisation and Part 2 the rest after the
 // per-step Householder kernels (k_hh_step, k_hh_finish).
-template <bool InLds, int Part = 0>
-__global__ void __launch_bounds__(InLds ? 256 : 1024) k_gep_lowest(const SlotDesc* __restrict__ slots, TopoDesc topo) {
+template <int Part>
+__global__ void __launch_bounds__(1024) k_gep_lowest(const SlotDesc* __restrict__ slots, TopoDesc topo) {
     const SlotDesc& sd = slots[blockIdx.z];
-    const auto Hs = to_global(sd.Hs);
-    const auto Ss = to_global(sd.Ss);
     const int n = topo.n_str;
     const double e_nuc = sd.e_nuc;
     double* __restrict__ gwork = sd.gep;
     const auto coef = to_global(sd.coef);
     const auto energy = to_global(sd.energy);
-    const auto flags = to_global(sd.flags);
     const long long* __restrict__ off = topo.off;
     const int* __restrict__ ts = topo.ts;
     const double* __restrict__ tc = topo.tc;
     const int n_det = topo.n_det;
     const auto dcoef = to_global(sd.dcoef);
-    extern __shared__ double lds[];
-    // LDS or device memory, typed as such so that neither instantiation uses flat accesses
-    const auto work = [&] {
-        if constexpr (InLds) return static_cast<double*>(lds);
-        else return to_global(gwork);
-    }();
+    const auto work = to_global(gwork);
     const auto Lm = work;              // n x n, lower Cholesky factor
     const auto M = work + n * n;       // n x n
     const auto V = work + 2 * n * n;   // Householder vectors (column k holds v_k)
@@ -1437,10 +1338,7 @@ __global__ void __launch_bounds__(InLds ? 256 : 1024) k_gep_lowest(const SlotDes
     const auto tdu = tdl + n;
     const auto tdu2 = tdu + n;
     const auto tdg = tdu2 + n;
-    const auto ipiv = [&] {  // n ints in the last n doubles
-        if constexpr (InLds) return reinterpret_cast<int*>(tdg + n);
-        else return reinterpret_cast<gptr<int>>(tdg + n);
-    }();
+    const auto ipiv = reinterpret_cast<gptr<int>>(tdg + n);  // n ints in the last n doubles
     __shared__ double red[16];
     __shared__ double sh_scalar[4];
     __shared__ double lo_hi[2];
@@ -1448,81 +1346,6 @@ __global__ void __launch_bounds__(InLds ? 256 : 1024) k_gep_lowest(const SlotDes
     const int tid = threadIdx.x, nt = blockDim.x;
     // 2D thread layout for element-parallel updates: TX consecutive lanes share a row
     const int TX = nt == 64 ? 8 : 16, TY = nt / TX, tx = tid % TX, ty = tid / TX;
-    if constexpr (Part == 0) {
-    for (int idx = tid; idx < n * n; idx += nt) {
-        const int i = idx % n, j = idx / n;
-        Lm[idx] = 0.5 * (Ss[i + n * j] + Ss[j + n * i]);
-        M[idx] = 0.5 * (Hs[i + n * j] + Hs[j + n * i]);
-        V[idx] = 0.0;
-    }
-    __syncthreads();
-    // Cholesky S = L L^T (right-looking; the lower triangle of Lm becomes L), trailing update
-    // spread over all threads element by element
-    for (int k = 0; k < n; ++k) {
-        const double a = Lm[k + n * k];
-        if (!(a > 0.0)) {
-            if (tid == 0) flags[FLAG_METRIC] = 1;
-            return;  // uniform: every thread read the same diagonal after the last barrier
-        }
-        const double dk = sqrt(a), rdk = 1.0 / dk;
-        __syncthreads();
-        for (int i = k + tid; i < n; i += nt) Lm[i + n * k] = (i == k) ? dk : Lm[i + n * k] * rdk;
-        __syncthreads();
-        for (int j = k + 1 + ty; j < n; j += TY) {  // column j, rows i >= j: consecutive lanes, consecutive i
-            const double ljk = Lm[j + n * k];
-            for (int i = j + tx; i < n; i += TX) Lm[i + n * j] -= Lm[i + n * k] * ljk;
-        }
-        __syncthreads();
-    }
-    // Linv = L^{-1} into V (lower triangle), one row per sweep: V[i,j] = -(sum_{k=j}^{i-1} L[i,k] V[k,j]) / L[i,i]
-    for (int i = 0; i < n; ++i) {
-        const double rl = 1.0 / Lm[i + n * i];
-        for (int j = tid; j <= i; j += nt) {
-            if (j == i) {
-                V[i + n * i] = rl;
-            } else {
-                double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-                int k = j;
-                for (; k + 3 < i; k += 4) {
-                    s0 += Lm[i + n * k] * V[k + n * j];
-                    s1 += Lm[i + n * (k + 1)] * V[k + 1 + n * j];
-                    s2 += Lm[i + n * (k + 2)] * V[k + 2 + n * j];
-                    s3 += Lm[i + n * (k + 3)] * V[k + 3 + n * j];
-                }
-                for (; k < i; ++k) s0 += Lm[i + n * k] * V[k + n * j];
-                V[i + n * j] = -((s0 + s1) + (s2 + s3)) * rl;
-            }
-        }
-        __syncthreads();
-    }
-    // standard form A = Linv H Linv^T: T1 = Linv H into Lm (L is not needed any more), A into M.
-    // Consecutive lanes take consecutive columns of one T1 row so that the trip count (i + 1) is
-    // uniform across them; H is symmetric, so H[k,j] is read as H[j,k] (unit stride across lanes).
-    for (int idx = tid; idx < n * n; idx += nt) {
-        const int j = idx % n, i = idx / n;
-        double s0 = 0.0, s1 = 0.0;
-        int k = 0;
-        for (; k + 1 <= i; k += 2) {
-            s0 += V[i + n * k] * M[j + n * k];
-            s1 += V[i + n * (k + 1)] * M[j + n * (k + 1)];
-        }
-        for (; k <= i; ++k) s0 += V[i + n * k] * M[j + n * k];
-        Lm[i + n * j] = s0 + s1;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < n * n; idx += nt) {
-        const int i = idx % n, j = idx / n;
-        double s0 = 0.0, s1 = 0.0;
-        int k = 0;
-        for (; k + 1 <= j; k += 2) {
-            s0 += Lm[i + n * k] * V[j + n * k];
-            s1 += Lm[i + n * (k + 1)] * V[j + n * (k + 1)];
-        }
-        for (; k <= j; ++k) s0 += Lm[i + n * k] * V[j + n * k];
-        M[idx] = s0 + s1;
-    }
-    __syncthreads();
-    }
     // symmetrise A; keep Linv in Lm (for c = Linv^T z at the end) and clear V for the reflectors
     if constexpr (Part != 2) {
     for (int idx = tid; idx < n * n; idx += nt) {
@@ -1543,7 +1366,7 @@ __global__ void __launch_bounds__(InLds ? 256 : 1024) k_gep_lowest(const SlotDes
     }
     if constexpr (Part == 1) return;
     // Householder tridiagonalisation: reflect rows/cols k+1..n-1 of column k
-    if constexpr (Part == 0 || Part == 3) {
+    if constexpr (Part == 3) {
     for (int k = 0; k < n - 2; ++k) {
         const int m0 = k + 1;
         double part = 0.0;
@@ -1752,7 +1575,7 @@ __global__ void __launch_bounds__(InLds ? 256 : 1024) k_gep_lowest(const SlotDes
 }
 
 // Selected states (state-averaged evaluations, workflow/evaluator.cpp:22-32,65-111): after the
-// global-memory dense solve (k_gep_lowest<false, 2 or 3>), whose workspace still holds L^-1 (Lm),
+// global-memory dense solve (k_gep_lowest<2 or 3>), whose workspace still holds L^-1 (Lm),
 // the Householder vectors and scalars (V, beta) and the tridiagonal (dd, ee), one workgroup per
 // problem finds eigenvalue state_idx[k] of the tridiagonal for each selected state by multisection
 // on Sturm counts (the smallest x with at least state_idx[k] + 1 eigenvalues below it), its vector
@@ -2140,7 +1963,6 @@ __global__ void k_normalization_pullback(const SlotDesc* __restrict__ slots) {
 // LDS of the pair kernels: full np x np kernel, S_act, h_act, per-wave group slabs and, for the
 // backward, the adjoint accumulators (full np x np when that still fits, else packed).
 constexpr size_t kPairLdsLimit = 160 * 1024;
-constexpr size_t kGepLdsLimit = 144 * 1024;
 constexpr unsigned kGepPerStepMax = 8;  // problems per launch up to which the large-n solve runs per step
 constexpr int kCholPerStepMinN = 256;   // below it one workgroup factors S faster than n launch pairs
 
@@ -2233,29 +2055,27 @@ hipError_t configure_kernels(int n, int ng, int n_str, int mmax) {
     if ((e = configure_ri_tiled()) != hipSuccess) return e;
     if ((e = configure_pairs_singular()) != hipSuccess) return e;
     if ((e = configure_strings()) != hipSuccess) return e;
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gep_lowest<true>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGepLdsLimit);
+    return configure_gep_large();
 }
 
-
-size_t gep_lds_bytes(int n) { return gep_core_doubles(n) * sizeof(double); }
-
-bool gep_in_lds(int n) { return gep_lds_bytes(n) <= kGepLdsLimit; }
 
 // Front half of the eigensolve in global memory: Cholesky S = L L^T (blocked over many workgroups
 // when per_step and the space is large, else one workgroup per problem), L^-1 and the standard-form
 // matrix A = L^-1 H L^-T. Workspace (SlotDesc::gep): L at 0, A at n^2, L^-1 column-major at 2 n^2.
 void launch_gep_front(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo, bool per_step) {
     const int ns = topo.n_str;
-    if (per_step && ns >= kCholPerStepMinN) {
+    // in LDS wherever the triangle fits (175 structures: 93 us; column by column in memory 557)
+    const bool in_lds = ns <= kCholLdsMaxN, blocked = per_step && !in_lds && ns >= kCholPerStepMinN;
+    if (in_lds || blocked)
         hipLaunchKernelGGL(k_gep_load, dim3((unsigned)(((long long)ns * ns + 255) / 256), 1, z), dim3(256), 0, st,
                            slots, ns);
+    if (in_lds) {
+        launch_gep_chol_lds(st, slots, z, ns);
+    } else if (blocked) {
         for (int j0 = 0; j0 < ns; j0 += kCholPanel) {
             const int jb = std::min(kCholPanel, ns - j0), rest = ns - j0 - jb;
-            hipLaunchKernelGGL(k_chol_diag, dim3(1, 1, z), dim3(256), 0, st, slots, ns, j0, jb);
+            launch_chol_panel(st, slots, z, ns, j0, jb);
             if (rest > 0) {
-                hipLaunchKernelGGL(k_chol_trsm, dim3((unsigned)((rest + 255) / 256), 1, z), dim3(256), 0, st, slots, ns,
-                                   j0, jb);
                 const unsigned tiles = (unsigned)((rest + 15) / 16);
                 hipLaunchKernelGGL(k_chol_syrk, dim3(tiles, tiles, z), dim3(256), 0, st, slots, ns, j0, jb);
             }
@@ -2263,10 +2083,7 @@ void launch_gep_front(hipStream_t st, const SlotDesc* slots, unsigned z, const T
     } else {
         hipLaunchKernelGGL(k_gep_chol, dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
     }
-    if (ns <= kLinvWaveMaxN)
-        hipLaunchKernelGGL(k_gep_linv, dim3((unsigned)((ns + 3) / 4), 1, z), dim3(256), 4 * (size_t)ns * sizeof(double),
-                           st, slots, ns);
-    else
+    if (!launch_gep_linv_cols(st, slots, z, ns))
         hipLaunchKernelGGL(k_gep_linv_lane, dim3((unsigned)((ns + 63) / 64), 1, z), dim3(64), 0, st, slots, ns);
     hipLaunchKernelGGL(k_gep_hlt, dim3((unsigned)((ns + 255) / 256), (unsigned)ns, z), dim3(256), 0, st, slots, ns);
     hipLaunchKernelGGL(k_gep_lul, dim3((unsigned)((ns + 255) / 256), (unsigned)ns, z), dim3(256), 0, st, slots, ns);
@@ -2361,34 +2178,31 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
     hipLaunchKernelGGL(k_structure_right, dim3((unsigned)((a + 255) / 256), 1, z), dim3(256), 0, st, slots, topo);
     hipLaunchKernelGGL(k_structure_left, dim3((unsigned)((b + 255) / 256), 1, z), dim3(256), 0, st, slots, topo);
     mark(EV_STRUCT);
-    const int threads = 256;
     // one selected state that is the lowest root: the lowest-root solvers; otherwise the
     // global-memory dense solve followed by the selected-states kernel
     const bool states = topo.n_states > 1 || topo.state_idx[0] != 0;
     if (shape.davidson)
         launch_davidson(st, slots, z, topo, shape);
     else if (!states && launch_gep_wave(st, slots, z, topo)) {
-    } else if (gep_in_lds(topo.n_str) && !states)
-        hipLaunchKernelGGL(k_gep_lowest<true>, dim3(1, 1, z), dim3(threads), gep_lds_bytes(topo.n_str), st, slots,
-                           topo);
-    else {
+    } else {
         // matrices in global memory: few problems per launch take the per-step Cholesky and
         // Householder kernels (many blocks each); batched launches keep one workgroup per problem
         // for those two stages, which the number of problems already parallelises
         const int ns = topo.n_str;
         const bool per_step = shape.pinned || z <= kGepPerStepMax;
         launch_gep_front(st, slots, z, topo, per_step);
-        if (per_step) {
-            hipLaunchKernelGGL((k_gep_lowest<false, 1>), dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
+        if (!states && launch_gep_lanczos(st, slots, z, topo)) {
+        } else if (per_step) {
+            hipLaunchKernelGGL((k_gep_lowest<1>), dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
             for (int k = 0; k + 2 < ns; ++k) {
                 const unsigned rows = (unsigned)((ns - (k + 1) + 3) / 4);
                 hipLaunchKernelGGL(k_hh_step, dim3(rows, 1, z), dim3(256), 3 * (size_t)ns * sizeof(double), st, slots,
                                    ns, k);
             }
             hipLaunchKernelGGL(k_hh_finish, dim3(1, 1, z), dim3(256), 2 * (size_t)ns * sizeof(double), st, slots, ns);
-            hipLaunchKernelGGL((k_gep_lowest<false, 2>), dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
+            hipLaunchKernelGGL((k_gep_lowest<2>), dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
         } else {
-            hipLaunchKernelGGL((k_gep_lowest<false, 3>), dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
+            hipLaunchKernelGGL((k_gep_lowest<3>), dim3(1, 1, z), dim3(1024), 0, st, slots, topo);
         }
         if (states) hipLaunchKernelGGL(k_gep_states, dim3(1, 1, z), dim3(256), 0, st, slots, topo);
     }

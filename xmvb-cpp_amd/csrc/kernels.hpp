@@ -189,11 +189,18 @@ void launch_pairs_singular(hipStream_t st, bool backward, int part_offset, const
 void launch_pairs_lane(hipStream_t st, int which, int blocks, const SlotDesc* slots, int count, const TopoDesc& topo,
                        int n_alpha, int n_beta, double cond_limit);
 bool pairs_full_dg(int n, int ng);
-std::size_t gep_lds_bytes(int n);
-bool gep_in_lds(int n);
 // Lowest root of one selected state for n_str <= 64: one wavefront per problem, columns in
 // registers (gep_wave.hip). Returns false, launching nothing, for larger structure spaces.
 bool launch_gep_wave(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+// Larger spaces (gep_large.hip): Cholesky with the metric in LDS, L^-1 by columns, and the lowest root of
+// A by Lanczos with full reorthogonalisation. Each returns false, launching nothing, beyond its size.
+constexpr int kCholPanel = 32;  // columns per panel of the blocked Cholesky
+void launch_chol_panel(hipStream_t st, const SlotDesc* slots, unsigned z, int n, int j0, int jb);
+constexpr int kCholLdsMaxN = 190;  // packed lower triangle of the metric: 145 KB of LDS
+void launch_gep_chol_lds(hipStream_t st, const SlotDesc* slots, unsigned z, int n);
+bool launch_gep_linv_cols(hipStream_t st, const SlotDesc* slots, unsigned z, int n);
+bool launch_gep_lanczos(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
+hipError_t configure_gep_large();
 hipError_t configure_kernels(int n, int ng, int n_str, int mmax);
 
 // A second stream for launches of few problems: kernels with disjoint outputs that each fill only
