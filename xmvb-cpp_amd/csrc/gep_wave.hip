@@ -1,5 +1,5 @@
-// One-wavefront dense eigensolve for small structure spaces (n_str <= 64): the lowest root of
-// H c = lambda S c with c^T S c = 1, GeneralizedEigensolver::solve_dense semantics
+// One-wavefront dense eigensolve for small structure spaces (n_str <= 64): the lowest root (or the
+// selected states) of H c = lambda S c with c^T S c = 1, GeneralizedEigensolver::solve_dense semantics
 // (linalg/eigensolver.cpp:365-387: Cholesky of the metric, standard form L^-1 H L^-T, lowest
 // eigenpair, c = L^-T z), and the determinant coefficients a_d = sum_I t_dI c_I.
 //
@@ -15,7 +15,8 @@
 //                    A <- (A + A^T) / 2 through another transpose
 //   tridiagonal:     Householder reflections, p = beta A v from lane j's own column (no cross-lane
 //                    sum), vectors kept in LDS (Wb) for the back-transform
-//   T y = lambda y:  tridiag_lowest_wave (multisection, inverse iteration, Rayleigh quotient)
+//   T y = lambda y:  tridiag_lowest_wave (multisection, inverse iteration, Rayleigh quotient), or
+//                    tridiag_state_wave for each selected state
 //   c = L^-T z:      backward substitution, c_k broadcast by readlane
 #include <hip/hip_runtime.h>
 
@@ -103,6 +104,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
     __shared__ double rl[N];               // 1 / L[k, k]
     __shared__ double hb[N];               // Householder beta
     __shared__ __align__(16) double tri[288];  // tridiagonal solver scratch
+    __shared__ double Zs[kMaxStates * 64];     // tridiagonal vectors of the states found
     const auto Ss = to_global(sd.Ss);
     const auto Hs = to_global(sd.Hs);
     double a[N];
@@ -246,36 +248,49 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
             }
         }
     }
-    double yv;
-    const double lambda = tridiag_lowest_wave(j, n, d_r, e_r, tri, yv);
-    for (int k = n - 3; k >= 0; --k) {  // back-transform z = H_0 H_1 ... H_{n-3} y
-        const double vk = j < N ? Wb[k * N + j] : 0.0;
-        yv -= hb[k] * wave_sum(vk * yv) * vk;
-    }
-    // c = L^-T z: c_k = (z_k - sum_{i > k} L[i, k] c_i) / L[k, k], z updated column by column
-    double c = 0.0, z = yv;
-    for (int k = n - 1; k >= 0; --k) {
-        const double ck = wave_bcast(z, k) * rl[k];
-        if (j == k) c = ck;
-        if (j < k) z -= Lc[j * N + k] * ck;
-    }
-    wave_sync();
-    if (j < n) {
-        to_global(sd.coef)[j] = c;
-        wv[j] = c;
+    const int states = topo.n_states;
+    const bool lowest = states == 1 && topo.state_idx[0] == 0;
+    double average = 0.0;
+    for (int s = 0; s < states; ++s) {
+        double yv;
+        const double lambda = lowest ? tridiag_lowest_wave(j, n, d_r, e_r, tri, yv)
+                                     : tridiag_state_wave(j, n, d_r, e_r, topo.state_idx[s], tri, Zs, s, yv);
+        if (!lowest) {
+            Zs[s * 64 + j] = yv;
+            wave_sync();
+        }
+        for (int k = n - 3; k >= 0; --k) {  // back-transform z = H_0 H_1 ... H_{n-3} y
+            const double vk = j < N ? Wb[k * N + j] : 0.0;
+            yv -= hb[k] * wave_sum(vk * yv) * vk;
+        }
+        // c = L^-T z: c_k = (z_k - sum_{i > k} L[i, k] c_i) / L[k, k], z updated column by column
+        double c = 0.0, z = yv;
+        for (int k = n - 1; k >= 0; --k) {
+            const double ck = wave_bcast(z, k) * rl[k];
+            if (j == k) c = ck;
+            if (j < k) z -= Lc[j * N + k] * ck;
+        }
+        wave_sync();
+        if (j < n) {
+            to_global(sd.coef)[(size_t)s * n + j] = c;
+            wv[j] = c;
+        }
+        average += lowest ? lambda : topo.state_w[s] * lambda;
+        if (j == 0 && !lowest) to_global(sd.state_energy)[s] = lambda;
+        wave_sync();
+        const auto off = to_global(topo.off);
+        const auto ts = to_global(topo.ts);
+        const auto tc = to_global(topo.tc);
+        for (int d = j; d < topo.n_det; d += 64) {
+            double acc = 0.0;
+            for (long long t = off[d]; t < off[d + 1]; ++t) acc += tc[t] * wv[ts[t]];
+            to_global(sd.dcoef)[(size_t)s * topo.n_det + d] = acc;
+        }
+        wave_sync();
     }
     if (j == 0) {
-        to_global(sd.energy)[0] = lambda;
-        to_global(sd.energy)[1] = lambda + sd.e_nuc;
-    }
-    wave_sync();
-    const auto off = to_global(topo.off);
-    const auto ts = to_global(topo.ts);
-    const auto tc = to_global(topo.tc);
-    for (int d = j; d < topo.n_det; d += 64) {
-        double acc = 0.0;
-        for (long long t = off[d]; t < off[d + 1]; ++t) acc += tc[t] * wv[ts[t]];
-        to_global(sd.dcoef)[d] = acc;
+        to_global(sd.energy)[0] = average;
+        to_global(sd.energy)[1] = average + sd.e_nuc;
     }
 }
 

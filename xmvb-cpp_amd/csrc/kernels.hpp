@@ -189,7 +189,7 @@ void launch_pairs_singular(hipStream_t st, bool backward, int part_offset, const
 void launch_pairs_lane(hipStream_t st, int which, int blocks, const SlotDesc* slots, int count, const TopoDesc& topo,
                        int n_alpha, int n_beta, double cond_limit);
 bool pairs_full_dg(int n, int ng);
-// Lowest root of one selected state for n_str <= 64: one wavefront per problem, columns in
+// Lowest root, or the selected states, for n_str <= 64: one wavefront per problem, columns in
 // registers (gep_wave.hip). Returns false, launching nothing, for larger structure spaces.
 bool launch_gep_wave(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
 // Larger spaces (gep_large.hip): Cholesky with the metric in LDS, L^-1 by columns, and the lowest root of

@@ -198,4 +198,98 @@ __device__ inline double tridiag_lowest_wave(int ln, int n, double d_r, double e
     return wave_sum(y * ty);
 }
 
+// Eigenpair `index` (ascending) of the same tridiagonal on one wavefront: multisection on Sturm counts to
+// rounding, then three steps of inverse iteration on T - lambda I (LU with partial pivoting as LAPACK's
+// dgttrf, row i's factors in lane i, the recurrences wave-uniform through readlane), each orthogonalised
+// against the `found` vectors of earlier states (Z[p 64 + i]), as dstein does within a cluster. t as in
+// tridiag_lowest_wave. Returns the Rayleigh quotient; yv receives the lane's component.
+__device__ inline double tridiag_state_wave(int ln, int n, double d_r, double e_r, int index, double* t, const double* Z,
+                                            int found, double& yv) {
+    double2* de = reinterpret_cast<double2*>(t);
+    const bool row = ln < n;
+    const double e_dn = __shfl_up(e_r, 1);
+    de[ln] = make_double2(row ? d_r : 0.0, ln > 0 && row ? e_dn * e_dn : 0.0);
+    if (ln < 8) de[64 + ln] = make_double2(0.0, 0.0);
+    const double rad = (ln > 0 && row ? fabs(e_dn) : 0.0) + fabs(e_r);
+    double lo = -wave_max(row ? rad - d_r : -1e300), hi = wave_max(row ? d_r + rad : -1e300);
+    const double pad = 1e-12 * fmax(fabs(lo), fabs(hi)) + 1e-300;
+    lo -= pad;
+    hi += pad;
+    wave_sync();
+    double unused = 0.0;
+    for (int it = 0; it < 64; ++it) {
+        if (!(hi - lo > 1e-15 * fmax(fabs(lo), fabs(hi)))) break;
+        const double x = lo + (hi - lo) * (double)(ln + 1) / 64.0;
+        const uint64_t hit = __ballot(sturm_count<false>(ln, n, de, x, unused) > index);
+        const int f = hit ? __builtin_ctzll(hit) : 64;
+        const double nlo = f == 0 ? lo : lo + (hi - lo) * (double)f / 64.0;
+        const double nhi = f >= 64 ? hi : lo + (hi - lo) * (double)(f + 1) / 64.0;
+        if (nlo == lo && nhi == hi) break;  // the points no longer separate
+        lo = nlo;
+        hi = nhi;
+    }
+    wave_sync();
+    const double lambda = 0.5 * (lo + hi);
+    double g = 1.0, u = 0.0, u2 = 0.0, l = 0.0, sw = 0.0;
+    {
+        double dc = wave_bcast(d_r, 0) - lambda, uc = n > 1 ? wave_bcast(e_r, 0) : 0.0;
+        for (int i = 0; i + 1 < n; ++i) {
+            const double dn = wave_bcast(d_r, i + 1) - lambda, li = wave_bcast(e_r, i);
+            const double un = i + 2 < n ? wave_bcast(e_r, i + 1) : 0.0;
+            if (fabs(dc) >= fabs(li)) {
+                const double piv = dc == 0.0 ? 1e-300 : dc, f = li / piv;
+                g = wave_put(piv, i, g);
+                u = wave_put(uc, i, u);
+                l = wave_put(f, i, l);
+                dc = dn - f * uc;
+                uc = un;
+            } else {
+                const double f = dc / li;
+                g = wave_put(li, i, g);
+                u = wave_put(dn, i, u);
+                u2 = wave_put(un, i, u2);
+                l = wave_put(f, i, l);
+                sw = wave_put(1.0, i, sw);
+                dc = uc - f * dn;
+                uc = -f * un;
+            }
+        }
+        g = wave_put(dc == 0.0 ? 1e-300 : dc, n - 1, g);
+    }
+    const double rg = 1.0 / g;
+    double y = row ? ((unsigned)(ln + 97 * found) * 2654435761u >> 31 ? -1.0 : 1.0) : 0.0;
+    for (int iter = 0; iter < 3; ++iter) {
+        double cur = wave_bcast(y, 0);
+        for (int i = 0; i + 1 < n; ++i) {
+            const double yn = wave_bcast(y, i + 1), li = wave_bcast(l, i);
+            if (wave_bcast(sw, i) == 0.0) {
+                y = wave_put(cur, i, y);
+                cur = yn - li * cur;
+            } else {
+                y = wave_put(yn, i, y);
+                cur = cur - li * yn;
+            }
+        }
+        y = wave_put(cur, n - 1, y);
+        double y1 = 0.0, y2 = 0.0;
+        for (int i = n - 1; i >= 0; --i) {
+            const double v = (wave_bcast(y, i) - wave_bcast(u, i) * y1 - wave_bcast(u2, i) * y2) * wave_bcast(rg, i);
+            y = wave_put(v, i, y);
+            y2 = y1;
+            y1 = v;
+        }
+        const double big = wave_max(fabs(y));
+        y *= big > 0.0 ? 1.0 / big : 1.0;  // squares of a nearly singular solve overflow
+        for (int p = 0; p < found; ++p) {
+            const double z = Z[p * 64 + ln];
+            y -= wave_sum(y * z) * z;
+        }
+        y *= 1.0 / sqrt(wave_sum(y * y));
+    }
+    const double y_dn = __shfl_up(y, 1), y_up = __shfl_down(y, 1);
+    const double ty = row ? d_r * y + (ln > 0 ? e_dn * y_dn : 0.0) + (ln + 1 < n ? e_r * y_up : 0.0) : 0.0;
+    yv = y;
+    return wave_sum(y * ty);
+}
+
 }  // namespace xmvb_amd
