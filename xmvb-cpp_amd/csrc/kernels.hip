@@ -853,8 +853,8 @@ __global__ void __launch_bounds__(256) k_reduce_partials_few(const SlotDesc* __r
 // pair and, when it has one, the spin-flip partner pair (the lane kernels defer the two together);
 // the count goes to FLAG_DEFERRED. Deferred == false: entries are the lane-group kernel's pairs (the
 // deferred list, or every pair when the shape has no lane kernel) and each flagged entry lists its
-// pair; the count goes to FLAG_SINGULAR_PAIRS. Three launches: per-chunk counts, their exclusive
-// scan (one block per slot), and the scatter, each chunk of kCompactChunk entries by one block.
+// pair; the count goes to FLAG_SINGULAR_PAIRS. For long lists three launches: per-chunk counts, their
+// exclusive scan (one block per slot), and the scatter, each chunk of kCompactChunk entries by one block.
 template <bool Deferred>
 struct CompactView {
     const uint8_t* flag;
@@ -972,12 +972,65 @@ __global__ void __launch_bounds__(kCompactChunk) k_compact_scatter(const SlotDes
     }
 }
 
+// The same list by one workgroup per slot in one launch, 8 flags per thread and sweep; launches bound it. Both
+// lists of 8,001 pairs (126 determinants) 9.1 us against 27.3 in six launches, of 31,878 pairs 8.7 against 19.6,
+// without the gaps between launches. Lists beyond four sweeps take the launches over many workgroups.
+constexpr int kCompactSweep = 8 * 1024;
+
+template <bool Deferred>
+__global__ void __launch_bounds__(1024) k_compact_few(const SlotDesc* __restrict__ slots, TopoDesc topo, int listed) {
+    const SlotDesc& sd = slots[blockIdx.z];
+    const CompactView<Deferred> v(sd, topo, listed);
+    __shared__ int wave_total[1024 / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const auto flag = to_global(v.flag);
+    int carry = 0;
+    for (long long base = 0; base < v.entries; base += kCompactSweep) {
+        const long long i0 = base + 8 * threadIdx.x;
+        unsigned long long set = 0;  // bit u: entry i0 + u is flagged
+        int count = 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (i0 + u < v.entries && flag[i0 + u]) set |= 1ull << u;
+        for (unsigned long long b = set; b; b &= b - 1) {
+            int first, second;
+            count += v.emit(sd, topo, listed, i0 + __builtin_ctzll(b), first, second);
+        }
+        int inclusive = count;  // over the wavefront
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(inclusive, off);
+            if (lane >= off) inclusive += y;
+        }
+        if (lane == 63) wave_total[wave] = inclusive;
+        __syncthreads();
+        int at = carry + inclusive - count;
+        for (int w = 0; w < 1024 / 64; ++w) {
+            if (w < wave) at += wave_total[w];
+            carry += wave_total[w];
+        }
+        for (unsigned long long b = set; b; b &= b - 1) {
+            int first = 0, second = 0;
+            const int c = v.emit(sd, topo, listed, i0 + __builtin_ctzll(b), first, second);
+            v.out[at] = first;
+            if (c == 2) v.out[at + 1] = second;
+            at += c;
+        }
+        __syncthreads();  // wave_total is read before the next sweep writes it
+    }
+    if (threadIdx.x == 0) to_global(sd.flags)[Deferred ? FLAG_DEFERRED : FLAG_SINGULAR_PAIRS] = carry;
+}
+
 // The deferred (Deferred) or rank-deficient list of every slot of a launch, in entry order. The
 // singular list's entry count is read on the device (the deferred count), so it runs after the
 // deferred list's kernels on the same stream.
 template <bool Deferred>
 void compact_pairs(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo, int listed,
                    long long max_entries) {
+    if (max_entries <= 4 * kCompactSweep) {
+        hipLaunchKernelGGL(k_compact_few<Deferred>, dim3(1, 1, z), dim3(1024), 0, st, slots, topo, listed);
+        return;
+    }
     const unsigned blocks = (unsigned)std::max<long long>(
         1, std::min<long long>(kCompactBlocks, (max_entries + kCompactChunk - 1) / kCompactChunk));
     hipLaunchKernelGGL(k_compact_count<Deferred>, dim3(blocks, 1, z), dim3(kCompactChunk), 0, st, slots, topo, listed);
