@@ -157,15 +157,27 @@ struct Slot {
     uint8_t* support_buf = nullptr;
 };
 
-// One stream with its descriptor table and compact per-launch outputs.
+// Energies (two) and flags of one slot of a launch.
+constexpr size_t kSlotOutBytes = 2 * sizeof(double) + FLAG_COUNT * sizeof(int);
+
+// One stream with its descriptor table and compact per-launch outputs. A launch of `count` slots lays its
+// energies, flags and descriptors out side by side on the device (the first two end where the descriptors
+// begin), so that cleared flags and descriptors go up in one copy and energies and flags come back in
+// one: a copy or a fill costs a launch, four of them about 20 us of the 250 us of the smallest calls.
 struct Lane {
     hipStream_t stream = nullptr;
+    unsigned char* d_table = nullptr;
+    unsigned char* h_table = nullptr;  // pinned: the image that goes up, then what comes back
     SlotDesc* d_desc = nullptr;
     SlotDesc* h_desc = nullptr;  // pinned
     double* d_energy = nullptr;
     int* d_flags = nullptr;
     double* h_energy = nullptr;  // pinned
     int* h_flags = nullptr;      // pinned
+    // a gradient that a single problem's launch also brings back, before its completion point
+    const double* back_src = nullptr;
+    double* back_dst = nullptr;  // pinned
+    size_t back_doubles = 0;
     double* d_C = nullptr;       // compact orbitals / gradients of submissions
     double* d_grad = nullptr;
     double* h_C = nullptr;       // pinned staging
@@ -183,6 +195,14 @@ struct Lane {
     int ticket = -1;
     std::vector<int> slots;
     std::vector<size_t> grad_offsets;
+
+    void lay_out(int capacity, int count) {
+        const size_t head = kSlotOutBytes * capacity;
+        d_energy = reinterpret_cast<double*>(d_table + head - kSlotOutBytes * count);
+        d_flags = reinterpret_cast<int*>(d_energy + 2 * count);
+        h_energy = reinterpret_cast<double*>(h_table + head + sizeof(SlotDesc) * capacity);
+        h_flags = reinterpret_cast<int*>(h_energy + 2 * count);
+    }
 };
 
 }  // namespace
@@ -228,9 +248,7 @@ struct vbe_pool {
             if (l.done) (void)hipEventDestroy(l.done);
             if (l.side.fork) (void)hipEventDestroy(l.side.fork);
             if (l.side.join) (void)hipEventDestroy(l.side.join);
-            if (l.h_desc) (void)hipHostFree(l.h_desc);
-            if (l.h_energy) (void)hipHostFree(l.h_energy);
-            if (l.h_flags) (void)hipHostFree(l.h_flags);
+            if (l.h_table) (void)hipHostFree(l.h_table);
             if (l.h_C) (void)hipHostFree(l.h_C);
             if (l.h_grad) (void)hipHostFree(l.h_grad);
         }
@@ -241,6 +259,12 @@ struct vbe_pool {
 struct vbe_problem {
     std::unique_ptr<vbe_pool> pool;
     bool forward_valid = false;
+    double* stage = nullptr;  // pinned: the orbitals of a host-buffer evaluation, then its gradient
+
+    ~vbe_problem() {
+        pool.reset();  // waits for the last launch
+        if (stage) (void)hipHostFree(stage);
+    }
 };
 
 namespace {
@@ -389,16 +413,12 @@ std::unique_ptr<vbe_pool> make_pool(vbe_context* ctx, const vbe_topology_view& t
         l.side.st = ctx->side_stream(l.stream);
         check(hipEventCreateWithFlags(&l.side.fork, hipEventDisableTiming), "hipEventCreate");
         check(hipEventCreateWithFlags(&l.side.join, hipEventDisableTiming), "hipEventCreate");
-        check(hipHostMalloc(reinterpret_cast<void**>(&l.h_desc), sizeof(SlotDesc) * capacity, hipHostMallocDefault),
-              "hipHostMalloc");
-        check(hipHostMalloc(reinterpret_cast<void**>(&l.h_energy), sizeof(double) * 2 * capacity, hipHostMallocDefault),
-              "hipHostMalloc");
-        check(hipHostMalloc(reinterpret_cast<void**>(&l.h_flags), sizeof(int) * FLAG_COUNT * capacity,
-                            hipHostMallocDefault),
-              "hipHostMalloc");
-        l.d_desc = p->topo_arena.alloc<SlotDesc>(capacity);
-        l.d_energy = p->topo_arena.alloc<double>(2 * (size_t)capacity);
-        l.d_flags = p->topo_arena.alloc<int>((size_t)FLAG_COUNT * capacity);
+        const size_t head = kSlotOutBytes * capacity, table = head + sizeof(SlotDesc) * capacity;
+        check(hipHostMalloc(reinterpret_cast<void**>(&l.h_table), table + head, hipHostMallocDefault), "hipHostMalloc");
+        l.d_table = p->topo_arena.alloc<unsigned char>(table);
+        l.h_desc = reinterpret_cast<SlotDesc*>(l.h_table + head);
+        l.d_desc = reinterpret_cast<SlotDesc*>(l.d_table + head);
+        l.lay_out(capacity, capacity);
     }
     hipStream_t st = p->lanes[0].stream;
     const int nd = t.n_determinants, ns = t.n_structures;
@@ -779,6 +799,7 @@ void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool wit
     const xmvb_amd::SideStream* side =
         lane.side.st != st && hipStreamQuery(lane.side.st) == hipSuccess ? &lane.side : nullptr;
     if (forward) {
+        lane.lay_out(p->capacity, count);
         std::vector<char> seen(p->capacity, 0);
         for (int i = 0; i < count; ++i) {
             const int s = in[i].slot;
@@ -796,8 +817,9 @@ void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool wit
             d.seeded = !ws && p->slots[s].has_root && p->ctx->dav_reuse_roots ? 1 : 0;
             lane.h_desc[i] = d;
         }
-        upload(lane.d_desc, lane.h_desc, count, st);
-        check(hipMemsetAsync(lane.d_flags, 0, sizeof(int) * FLAG_COUNT * count, st), "hipMemsetAsync");
+        const size_t flag_bytes = sizeof(int) * FLAG_COUNT * count, at = kSlotOutBytes * p->capacity - flag_bytes;
+        std::memset(lane.h_table + at, 0, flag_bytes);
+        upload(lane.d_table + at, lane.h_table + at, flag_bytes + sizeof(SlotDesc) * count, st);
         xmvb_amd::launch_forward(st, lane.d_desc, count, p->topo, sh, timed ? lane.ev : nullptr, side);
         check(hipGetLastError(), "forward launch");
     }
@@ -805,10 +827,11 @@ void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool wit
         xmvb_amd::launch_backward(st, lane.d_desc, count, p->topo, sh, timed ? lane.ev : nullptr, side);
         check(hipGetLastError(), "backward launch");
     }
-    check(hipMemcpyAsync(lane.h_energy, lane.d_energy, sizeof(double) * 2 * count, hipMemcpyDeviceToHost, st),
-          "energy D2H");
-    check(hipMemcpyAsync(lane.h_flags, lane.d_flags, sizeof(int) * FLAG_COUNT * count, hipMemcpyDeviceToHost, st),
-          "flags D2H");
+    check(hipMemcpyAsync(lane.h_energy, lane.d_energy, kSlotOutBytes * count, hipMemcpyDeviceToHost, st),
+          "energies and flags D2H");
+    if (with_grad && lane.back_doubles)
+        check(hipMemcpyAsync(lane.back_dst, lane.back_src, lane.back_doubles * sizeof(double), hipMemcpyDeviceToHost, st),
+              "gradient D2H");
     // the lane's completion point (the stream may carry other pools' launches after it)
     check(hipEventRecord(lane.done, st), "hipEventRecord");
     lane.slots.clear();
@@ -936,24 +959,33 @@ void check_flags_args(const vbe_flags& flags, const vbe_pool* p) {
         throw StatusError(VBE_ERR_ARGUMENT, "unknown eigensolver");
 }
 
-// Evaluate slot 0 of a single problem synchronously; C/support/grad are device pointers.
+// Evaluate slot 0 of a single problem synchronously; C/support/grad are device pointers. host_grad (optional)
+// receives the gradient, which comes back with the launch through pinned memory: one wait instead of two.
 double eval_problem(vbe_problem* prob, const double* d_C, const uint8_t* d_support, bool want_grad, double* d_grad,
-                    bool forward) {
+                    bool forward, double* host_grad = nullptr) {
     vbe_pool* p = prob->pool.get();
     check(hipSetDevice(p->ctx->device), "hipSetDevice");
     Lane& lane = p->lanes[0];
     std::vector<SlotInput> in{{0, d_C, d_support, d_grad}};
     if (forward) prob->forward_valid = false;
+    const size_t nc = (size_t)p->n_act * p->slots[0].n_bf;
     lane.busy = true;
+    lane.back_src = d_grad;
+    lane.back_dst = prob->stage + nc;
+    lane.back_doubles = want_grad && host_grad ? nc : 0;
     try {
         // a single problem's launch shape is the pinned one (the same bits as in any pinned batch)
         evaluate_now(p, lane, in, want_grad, forward, nullptr, true);
     } catch (...) {
+        lane.back_doubles = 0;
         lane.busy = false;
         throw;
     }
+    const bool back = lane.back_doubles != 0;
+    lane.back_doubles = 0;
     finish(p, lane);
     prob->forward_valid = true;
+    if (back) std::memcpy(host_grad, prob->stage + nc, nc * sizeof(double));
     return lane.h_energy[1];
 }
 
@@ -1550,6 +1582,9 @@ int vbe_problem_upload(vbe_context* ctx, const vbe_dims* dims, const double* S_a
         auto prob = std::make_unique<vbe_problem>();
         prob->pool = make_pool(ctx, *topo, dims->n_act, dims->n_alpha, dims->n_beta, 1);
         load_slot(prob->pool.get(), 0, dims->n_bf, dims->n_aux, S_ao, h_ao, B_packed, e_nuc);
+        check(hipHostMalloc(reinterpret_cast<void**>(&prob->stage), 2 * sizeof(double) * dims->n_act * dims->n_bf,
+                            hipHostMallocDefault),
+              "hipHostMalloc");
         *out = prob.release();
         return VBE_OK;
     });
@@ -1575,15 +1610,12 @@ int vbe_eval(vbe_context* ctx, vbe_problem* prob, const double* C_raw, const uin
         const size_t nc = (size_t)p->n_act * s.n_bf;
         hipStream_t st = p->lanes[0].stream;
         check(hipSetDevice(ctx->device), "hipSetDevice");
-        upload(s.C_buf, C_raw, nc, st);
+        std::memcpy(prob->stage, C_raw, nc * sizeof(double));
+        upload(s.C_buf, prob->stage, nc, st);
         if (support) upload(s.support_buf, support, nc, st);
         *E_total = eval_problem(prob, s.C_buf, support ? s.support_buf : nullptr, flags.want_gradient != 0,
-                                s.grad_buf, true);
+                                s.grad_buf, true, grad_raw);
         if (E_states) E_states[0] = *E_total;
-        if (flags.want_gradient) {
-            check(hipMemcpyAsync(grad_raw, s.grad_buf, nc * sizeof(double), hipMemcpyDeviceToHost, st), "gradient D2H");
-            check(hipStreamSynchronize(st), "hipStreamSynchronize");
-        }
         return VBE_OK;
     });
 }
@@ -1619,11 +1651,7 @@ int vbe_complete_gradient(vbe_context* ctx, vbe_problem* prob, double* grad_raw)
         // host-buffer evaluations
         p->lanes[0].h_desc[0].grad = s.grad_buf;
         upload(p->lanes[0].d_desc, p->lanes[0].h_desc, 1, p->lanes[0].stream);
-        eval_problem(prob, s.C_buf, p->lanes[0].h_desc[0].support, true, s.grad_buf, false);
-        const size_t nc = (size_t)p->n_act * s.n_bf;
-        hipStream_t st = p->lanes[0].stream;
-        check(hipMemcpyAsync(grad_raw, s.grad_buf, nc * sizeof(double), hipMemcpyDeviceToHost, st), "gradient D2H");
-        check(hipStreamSynchronize(st), "hipStreamSynchronize");
+        eval_problem(prob, s.C_buf, p->lanes[0].h_desc[0].support, true, s.grad_buf, false, grad_raw);
         return VBE_OK;
     });
 }
