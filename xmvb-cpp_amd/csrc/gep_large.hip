@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(256) k_gep_linv_cols(const SlotDesc* __restric
         x[r] = lane + 64 * r == j ? 1.0 : 0.0;
         rd[r] = 1.0 / L[i + (size_t)n * i];
     }
-    constexpr int kAhead = R <= 4 ? 8 : R <= 7 ? 4 : 2;
+    constexpr int kAhead = R <= 4 ? 8 : R <= 7 ? 4 : R <= 16 ? 2 : 1;
     auto fetch = [&](double (&c)[kAhead][R], int k0) {
 #pragma unroll
         for (int u = 0; u < kAhead; ++u)
@@ -625,6 +625,7 @@ bool launch_gep_linv_cols(hipStream_t st, const SlotDesc* slots, unsigned z, int
     else if (n <= 256) hipLaunchKernelGGL(k_gep_linv_cols<4>, grid, block, 0, st, slots, n);
     else if (n <= 448) hipLaunchKernelGGL(k_gep_linv_cols<7>, grid, block, 0, st, slots, n);
     else if (n <= 1024) hipLaunchKernelGGL(k_gep_linv_cols<16>, grid, block, 0, st, slots, n);
+    else if (n <= 2048) hipLaunchKernelGGL(k_gep_linv_cols<32>, grid, block, 0, st, slots, n);
     else return false;
     return true;
 }
