@@ -234,7 +234,7 @@ struct vbe_pool {
     // forward one-pair-per-lane blocks (the lane-group kernel takes twice this), backward blocks
     int fwd_target = kLaneBlocks;
     int bwd_target = kLaneBlocks;
-    int pair_hold = 0;  // launches left that include the pair kernels from the start (evaluate_now)
+    int pair_hold = 1;  // launches left that include the pair kernels from the start (evaluate_now)
 
     // serializes host access to the pool's lanes and slots between the caller's thread and the
     // request scheduler's dispatcher thread
@@ -902,27 +902,26 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
     if (status != VBE_OK && !slot_status) throw StatusError(status, err);
 }
 
-// A launch that the caller waits for at once: the string form alone first, without the idle launches of the
-// pair kernels (fourteen, 50-60 us of a 510 us evaluation of 252 determinants). Should a slot turn
-// out to need them (S_act too ill-conditioned, or a block that may be rank deficient), the launch is
-// repeated with them, and the pool's next kPairHold launches start with them.
+// A launch that the caller waits for at once: the string form alone, without the idle launches of the pair
+// kernels (fourteen, 50-60 us of a 510 us evaluation of 252 determinants), once a launch of the pool has shown
+// that no slot needs them (S_act too ill-conditioned, or a block that may be rank deficient). Should a
+// slot then turn out to need them, the launch is repeated with them, and the pool takes both until
+// kPairHold launches in a row have needed none.
 constexpr int kPairHold = 64;
 void evaluate_now(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
                   const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true) {
     // a repeated Davidson solve would start from what the first one left
     const bool strings_only = forward && p->pair_hold == 0 && p->eigensolver != VBE_EIGENSOLVER_DAVIDSON;
-    if (forward && p->pair_hold > 0) --p->pair_hold;
     enqueue(p, lane, in, with_grad, forward, ws, pinned, timed, strings_only);
-    if (!forward || lane.pair_kernels) return;
+    if (!forward || !lane.strings) return;
     check(hipEventSynchronize(lane.done), "hipEventSynchronize");
     bool left = false;
     for (size_t i = 0; i < in.size(); ++i) {
         const int* f = lane.h_flags + FLAG_COUNT * i;
         left = left || !f[xmvb_amd::FLAG_STRINGS] || f[xmvb_amd::FLAG_NEAR];
     }
-    if (!left) return;
-    p->pair_hold = kPairHold;
-    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed);
+    p->pair_hold = left ? kPairHold : std::max(p->pair_hold - 1, 0);
+    if (left && !lane.pair_kernels) enqueue(p, lane, in, with_grad, forward, ws, pinned, timed);
 }
 
 Lane& acquire_lane(vbe_pool* p) {
