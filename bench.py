@@ -22,7 +22,7 @@ Three legs are timed:
     iteration next to the plain evaluation time.
 
 Prints one JSON line: batched throughput (E+grad evaluations/s) beside the plain path's, request
-p50/p99 latency of the served leg, the roofline of the dominant pair kernel of the batched leg (its
+p50/p99 latency of the served leg, the roofline of the longest single kernel of the batched leg (its
 duration from HIP events recorded on the engine stream during the timed region), parity against
 the FP64 CPU oracle and the oracle's own throughput on the host cores (cpu_baseline).
 """
@@ -417,6 +417,14 @@ def main():
         "k_gep_wave": (mean["eigensolve_ms"], "mfma", K * 10.0 * topo.n_structures ** 3, "TFLOP/s",
                        "latency: per-step LDS round trips, wave reductions and serial recurrences"),
     }
+    # the determinant strings replace the pair kernels where every slot allows it (nothing then runs between the
+    # events around the pair kernels' adjoint): several kernels each way, reported as phases without a roofline
+    strings = mean["pair_backward_adjoint_ms"] < 0.05 * mean["pair_backward_field_ms"]
+    if strings:
+        kernels = {k: v for k, v in kernels.items() if not k.startswith("k_pairs_lane")}
+    determinant_form = dict(form="strings" if strings else "pairs", forward_ms=mean["pair_forward_ms"],
+                            backward_ms=mean["pair_backward_ms"],
+                            pairwise_flops_per_direction=f_det)
     traffic_table = {}
     if os.path.exists(TRAFFIC_FILE):
         with open(TRAFFIC_FILE) as f:
@@ -693,7 +701,8 @@ def main():
                served_mixed_sizes=served_mixed, mixed_precision=mixed, precision_form=precision,
                converge=converge, mixed_batch=mixed_batch,
                batch_consistency=batch_consistency, phase_ms={k: round(v, 5) for k, v in mean.items()},
-               energy=energy, roofline=roofline, roofline_other_kernels=others)
+               energy=energy, determinant_form=determinant_form, roofline=roofline,
+               roofline_other_kernels=others)
     if not args.no_cpu:
         base, parity = cpu_baseline(cfg, sp, topo, energy, grad, args.cpu_seconds)
         out["cpu_baseline"] = base

@@ -202,7 +202,8 @@ int vbe_last_error(const vbe_context* ctx, char* buf, size_t len);
  * overlap.cpp:50-110) directly. Any limit in [0, 1e9] keeps results within rounding of the
  * reference (below 1e9 a row-pivoted block is provably full rank under that rule); 0 sends every
  * pair through the complete-pivoting path. Default 1e5: worse-conditioned blocks then follow the
- * reference's pivot order, which keeps their rounding close to it. Applies to later evaluations.
+ * reference's pivot order, which keeps their rounding close to it; at the default the pairs may also
+ * be evaluated over determinant strings where S_act is well conditioned. Applies to later evaluations.
  * No counterpart in the reference, which has a single (CPU) pair path. */
 int vbe_set_pair_condition_limit(vbe_context* ctx, double limit);
 /* Storage precision of the RI factors for problems and pools created after the call

@@ -193,7 +193,7 @@ bool pairs_full_dg(int n, int ng);
 // registers (gep_wave.hip). Returns false, launching nothing, for larger structure spaces.
 bool launch_gep_wave(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
 // Larger spaces (gep_large.hip): Cholesky with the metric in LDS, L^-1 by columns, and the lowest root of
-// A by Lanczos with full reorthogonalisation. Each returns false, launching nothing, beyond its size.
+// A by Lanczos with full reorthogonalisation. Those that return false launch nothing: beyond their size.
 constexpr int kCholPanel = 32;  // columns per panel of the blocked Cholesky
 void launch_chol_panel(hipStream_t st, const SlotDesc* slots, unsigned z, int n, int j0, int jb);
 constexpr int kCholLdsMaxN = 190;  // packed lower triangle of the metric: 145 KB of LDS
