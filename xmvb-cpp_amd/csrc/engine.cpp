@@ -190,7 +190,8 @@ struct Lane {
     bool with_grad = false;
     bool events_valid = false;
     bool strings = false;       // the last forward offered the string form
-    bool pair_kernels = true;   // and launched the pair kernels beside it
+    bool string_kernels = false;  // and launched its kernels
+    bool pair_kernels = true;     // and the pair kernels
     bool scratch = false;  // the launch ran on a workspace outside the slots (no-allocation entry point)
     int ticket = -1;
     std::vector<int> slots;
@@ -235,6 +236,7 @@ struct vbe_pool {
     int fwd_target = kLaneBlocks;
     int bwd_target = kLaneBlocks;
     int pair_hold = 1;  // launches left that include the pair kernels from the start (evaluate_now)
+    int pair_run = 0;   // launches in a row that no slot's string form served; below zero: launches to wait first
 
     // serializes host access to the pool's lanes and slots between the caller's thread and the
     // request scheduler's dispatcher thread
@@ -774,13 +776,15 @@ LaunchShape shape_for(const vbe_pool* p, const std::vector<SlotInput>& in, bool 
     return sh;
 }
 
+enum class Forms { both, strings, pairs };
+
 // Enqueue forward and/or backward for a set of slots on a lane, then the D2H of energies and flags.
 // ws (optional, single-slot launches): a descriptor whose workspace replaces the slot's own.
-// strings_only: where the string form is offered, leave the pair kernels out (see evaluate_now).
+// forms: where the string form is offered, the kernels of both forms, or of one of them (see evaluate_now).
 // timed: record the phase events (read by finish into the pool's phase times); the optimiser's
 // inner evaluations skip them, a dozen event records per launch being host time on its critical path.
 void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
-             const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true, bool strings_only = false) {
+             const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true, Forms forms = Forms::both) {
     const int count = (int)in.size();
     if (count <= 0 || count > p->capacity) throw StatusError(VBE_ERR_ARGUMENT, "invalid number of slots");
     if (ws && count != 1) throw StatusError(VBE_ERR_ARGUMENT, "a replacement workspace serves one slot");
@@ -790,10 +794,12 @@ void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool wit
     // the gradient of an earlier forward follows the form that forward took
     if (forward) {
         lane.strings = sh.strings;
-        lane.pair_kernels = !sh.strings || !strings_only;
+        lane.string_kernels = sh.strings && forms != Forms::pairs;
+        lane.pair_kernels = !sh.strings || forms != Forms::strings;
     } else {
         sh.strings = lane.strings;
     }
+    sh.string_kernels = lane.string_kernels;
     sh.pair_kernels = lane.pair_kernels;
     // the side stream only when it is idle: queued behind another lane's launch it would delay this one
     const xmvb_amd::SideStream* side =
@@ -906,22 +912,33 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
 // kernels (fourteen, 50-60 us of a 510 us evaluation of 252 determinants), once a launch of the pool has shown
 // that no slot needs them (S_act too ill-conditioned, or a block that may be rank deficient). Should a
 // slot then turn out to need them, the launch is repeated with them, and the pool takes both until
-// kPairHold launches in a row have needed none.
-constexpr int kPairHold = 64;
+// kPairHold launches in a row have needed none. Where kPairRun launches in a row had no slot for the
+// string form at all, its kernels stay out in turn, but for the test of S_act: a slot that passes it has the launch
+// repeated. The form of a slot follows from its own S_act in every case.
+constexpr int kPairHold = 64, kPairRun = 4;
 void evaluate_now(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
                   const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true) {
     // a repeated Davidson solve would start from what the first one left
-    const bool strings_only = forward && p->pair_hold == 0 && p->eigensolver != VBE_EIGENSOLVER_DAVIDSON;
-    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed, strings_only);
+    const bool davidson = p->eigensolver == VBE_EIGENSOLVER_DAVIDSON;
+    const Forms forms = !forward || davidson     ? Forms::both
+                        : p->pair_run >= kPairRun ? Forms::pairs
+                        : p->pair_hold == 0       ? Forms::strings
+                                                  : Forms::both;
+    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed, forms);
     if (!forward || !lane.strings) return;
     check(hipEventSynchronize(lane.done), "hipEventSynchronize");
-    bool left = false;
+    bool pairs = false, strings = false;
     for (size_t i = 0; i < in.size(); ++i) {
         const int* f = lane.h_flags + FLAG_COUNT * i;
-        left = left || !f[xmvb_amd::FLAG_STRINGS] || f[xmvb_amd::FLAG_NEAR];
+        strings = strings || f[xmvb_amd::FLAG_STRINGS];
+        pairs = pairs || !f[xmvb_amd::FLAG_STRINGS] || f[xmvb_amd::FLAG_NEAR];
     }
-    p->pair_hold = left ? kPairHold : std::max(p->pair_hold - 1, 0);
-    if (left && !lane.pair_kernels) enqueue(p, lane, in, with_grad, forward, ws, pinned, timed);
+    p->pair_hold = pairs ? kPairHold : std::max(p->pair_hold - 1, 0);
+    const bool missing = (strings && !lane.string_kernels) || (pairs && !lane.pair_kernels);
+    p->pair_run = !strings                    ? p->pair_run + (p->pair_run < kPairRun)
+                  : forms == Forms::pairs     ? -kPairHold
+                                              : std::min(p->pair_run, 0);
+    if (missing) enqueue(p, lane, in, with_grad, forward, ws, pinned, timed);
 }
 
 Lane& acquire_lane(vbe_pool* p) {

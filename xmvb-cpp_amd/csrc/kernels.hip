@@ -2162,7 +2162,7 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
     hipLaunchKernelGGL(k_active_matrices, dim3(1, 1, z), dim3(256), 0, active, slots, n);
     if (shape.strings) {
         launch_string_frame(active, slots, z, topo);
-        launch_string_minors(active, slots, z, topo);
+        if (shape.string_kernels) launch_string_minors(active, slots, z, topo);
     }
     if (fork) (void)hipEventRecord(side->join, side->st);
     mark(EV_PREP);
@@ -2206,14 +2206,14 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
     if (fork) (void)hipStreamWaitEvent(st, side->join, 0);
     mark(EV_TRANSFORM);
     const long long all_pairs = (long long)topo.n_det * (topo.n_det + 1) / 2;
-    if (shape.strings) {
+    if (shape.string_kernels) {
         launch_string_integrals(st, slots, z, topo);
         launch_string_forward(st, slots, z, topo);
     }
     if (!shape.pair_kernels) {
         mark(EV_PAIR_FWD_MAIN);
     } else if (shape.lane_fwd) {
-        if (shape.strings) launch_string_defer(st, slots, z, topo);
+        if (shape.string_kernels) launch_string_defer(st, slots, z, topo);
         launch_pairs_lane(st, 0, shape.lane_blocks_fwd, slots, count, topo, shape.n_alpha, shape.n_beta,
                           shape.lane_cond_limit);
         mark(EV_PAIR_FWD_MAIN);
@@ -2271,14 +2271,14 @@ void launch_backward(hipStream_t st, const SlotDesc* slots, int count, const Top
         if (ev) (void)hipEventRecord(ev[k], st);
     };
     mark(EV_BWD_BEGIN);
-    if (shape.strings) launch_string_backward(st, slots, z, topo);
+    if (shape.string_kernels) launch_string_backward(st, slots, z, topo);
     if (!shape.pair_kernels) {
         for (const int k : {EV_BWD_FIELD, EV_BWD_ADJOINT, EV_BWD_KERNEL}) mark(k);
     } else {
         // The pair-adjoint kernels write disjoint columns (field: ds/dh; adjoint: dg) or disjoint rows
         // (deferred list, singular pairs) of the partial rows, so for few problems the adjoint kernel and
         // the singular-pair kernel run on the side stream beside the field and deferred-list kernels.
-        const bool fork = side && count <= kForkMaxProblems && shape.lane_bwd && !shape.strings;
+        const bool fork = side && count <= kForkMaxProblems && shape.lane_bwd && !shape.string_kernels;
         hipStream_t st2 = st;
         if (fork) {
             (void)hipEventRecord(side->fork, st);

@@ -117,6 +117,7 @@ struct LaunchShape {
     bool any_tiled, any_flat;              // slots of the launch with the aux-tiled / the flat layout
     int max_n_bf_tiled;                    // largest n_bf among the slots with the aux-tiled layout
     bool strings;                          // slots may take the string form (their FLAG_STRINGS decides)
+    bool string_kernels;                   // launch the string form's kernels (else only the test of S_act)
     bool pair_kernels;                     // launch the pair kernels too, for slots or pairs the string form leaves
     bool davidson;                         // structure eigenproblem by Davidson instead of dense
     // Pinned launch shape: every choice that changes a slot's summation order (blocks per slot of the
