@@ -33,9 +33,13 @@ __device__ __forceinline__ void problem_block(int& x, int& z) {
     x = (int)(k % nx);
 }
 
-// The slot's determinant pairs are evaluated in the string form (strings.hip): the pair kernels of the
-// same launch leave it alone. Uniform over a launch's workgroups of a slot.
-__device__ __forceinline__ bool string_slot(const SlotDesc& sd) { return to_global(sd.flags)[FLAG_STRINGS] != 0; }
+// The slot's determinant pairs are evaluated in the string form (strings.hip), but for its listed pairs: the lane
+// kernels of the same launch leave it alone. Uniform over a launch's workgroups of a slot (FLAG_NEAR
+// is complete before the first kernel that asks, other than those that set it).
+__device__ __forceinline__ bool string_slot(const SlotDesc& sd) {
+    const auto f = to_global(sd.flags);
+    return f[FLAG_STRINGS] != 0 && f[FLAG_NEAR] <= kStringListMax;
+}
 
 // unordered pair t = e(e+1)/2 + d with d <= e
 __device__ __forceinline__ void unpack_pair(long long t, int& d, int& e) {

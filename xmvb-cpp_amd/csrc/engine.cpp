@@ -554,8 +554,9 @@ void check_slots_free(const vbe_pool* p, const int* slots, int count) {
 // Per-evaluation workspace of one slot of a pool, carved from one block of device memory (arrays
 // aligned to 256 bytes). With base == nullptr nothing is assigned and only the size is returned.
 // The slot's own arena and the no-allocation entry point's static scratch use this same layout.
-// The string form's arrays lie over the pair kernels' partial rows where they fit (a slot uses one
-// or the other), else behind everything else; strings = false leaves them out.
+// The string form's arrays lie over the partial rows of the lane kernels where they fit (a slot uses one
+// or the other; the front rows hold the listed pairs'), else behind everything else; strings = false
+// leaves them out.
 size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* base, SlotDesc& d, bool strings = true) {
     const TopoDesc& T = p->topo;
     const size_t n = T.n, np = T.np, nd = T.n_det, ns = T.n_str;
@@ -602,8 +603,9 @@ size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* ba
     if (strings && T.str.enabled) {
         xmvb_amd::StringWork unused{};
         const size_t count = xmvb_amd::string_work_carve(T, nullptr, unused);
-        double* work = d.partials;
-        if (count > partial_rows) take(work, count);
+        const size_t front = ((size_t)(xmvb_amd::kListBlocks + xmvb_amd::kSingularBlocks) * len + 31) / 32 * 32;
+        double* work = base ? d.partials + front : nullptr;
+        if (front + count > partial_rows) take(work, count);
         if (base) (void)xmvb_amd::string_work_carve(T, work, d.sw);
     }
     return (off + 255) & ~size_t(255);
@@ -908,9 +910,9 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
     if (status != VBE_OK && !slot_status) throw StatusError(status, err);
 }
 
-// A launch that the caller waits for at once: the string form alone, without the idle launches of the pair
-// kernels (fourteen, 50-60 us of a 510 us evaluation of 252 determinants), once a launch of the pool has shown
-// that no slot needs them (S_act too ill-conditioned, or a block that may be rank deficient). Should a
+// A launch that the caller waits for at once: the string form and the list kernels alone, without the idle launches
+// of the lane kernels, once a launch of the pool has shown that no slot needs them (S_act too ill-conditioned,
+// or too many listed pairs). Should a
 // slot then turn out to need them, the launch is repeated with them, and the pool takes both until
 // kPairHold launches in a row have needed none. Where kPairRun launches in a row had no slot for the
 // string form at all, its kernels stay out in turn, but for the test of S_act: a slot that passes it has the launch
@@ -930,8 +932,9 @@ void evaluate_now(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, boo
     bool pairs = false, strings = false;
     for (size_t i = 0; i < in.size(); ++i) {
         const int* f = lane.h_flags + FLAG_COUNT * i;
-        strings = strings || f[xmvb_amd::FLAG_STRINGS];
-        pairs = pairs || !f[xmvb_amd::FLAG_STRINGS] || f[xmvb_amd::FLAG_NEAR];
+        const bool string_slot = f[xmvb_amd::FLAG_STRINGS] && f[xmvb_amd::FLAG_NEAR] <= xmvb_amd::kStringListMax;
+        strings = strings || string_slot;
+        pairs = pairs || !string_slot;
     }
     p->pair_hold = pairs ? kPairHold : std::max(p->pair_hold - 1, 0);
     const bool missing = (strings && !lane.string_kernels) || (pairs && !lane.pair_kernels);

@@ -540,7 +540,6 @@ __global__ void __launch_bounds__(512) k_pairs(const SlotDesc* __restrict__ slot
     constexpr int MB = GroupShape<GROUP>::MB;
     constexpr int GPW = 64 / GROUP;  // groups per wavefront
     const SlotDesc& sd = slots[blockIdx.z];
-    if (Backward && string_slot(sd)) return;
     const auto G_glob = to_global(sd.G);
     const int n = topo.n, ng = topo.ng, n_det = topo.n_det;
     const int np = n * (n + 1) / 2;
@@ -785,7 +784,7 @@ __global__ void __launch_bounds__(512) k_pairs(const SlotDesc* __restrict__ slot
     if (Backward) {
         __syncthreads();
         const int stride_part = ng + 2 * n * n;
-        double* out = sd.partials + (size_t)(blockIdx.x + part_offset) * stride_part;
+        double* out = sd.partials + (size_t)(blockIdx.x + (string_slot(sd) ? 0 : part_offset)) * stride_part;
         if (FullDg) {
             for (int t = threadIdx.x; t < ng; t += blockDim.x) {
                 int Q, P;
@@ -804,11 +803,26 @@ __global__ void __launch_bounds__(512) k_pairs(const SlotDesc* __restrict__ slot
 
 // sum block partials in a fixed order: out[i] = sum_b partials[b*len + i], one wavefront per i.
 // Rows [list_begin, list_begin + list_rows) belong to the deferred-list blocks, which take
-// list_per_row pairs per sweep; a row whose block had no pair was not written and is skipped.
+// list_per_row pairs per sweep; a row whose block had no pair was not written and is skipped. A string slot
+// has rows of its listed pairs alone, at the front (kListBlocks, then the singular pairs'), and adds them to
+// the strings' own sum.
+struct PartialRows {
+    int rows, list_begin;
+    bool strings;
+    __device__ PartialRows(const SlotDesc& sd, int n_blocks, int begin, int list_rows)
+        : rows(n_blocks), list_begin(begin), strings(string_slot(sd)) {
+        if (strings) {
+            rows = list_rows + kSingularBlocks;
+            list_begin = 0;
+        }
+    }
+    __device__ size_t at(int b, int list_rows) const { return strings && b >= list_rows ? b - list_rows + kListBlocks : b; }
+};
+
 __global__ void k_reduce_partials(const SlotDesc* __restrict__ slots, int n_blocks, int len, int list_begin,
                                   int list_rows, int list_per_row) {
     const SlotDesc& sd = slots[blockIdx.z];
-    if (string_slot(sd)) return;
+    const PartialRows p(sd, n_blocks, list_begin, list_rows);
     const auto partials = to_global(sd.partials);
     const auto out = to_global(sd.dsum);
     const int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -816,13 +830,13 @@ __global__ void k_reduce_partials(const SlotDesc* __restrict__ slots, int n_bloc
     if (i >= len) return;
     const long long deferred = list_rows > 0 ? (long long)to_global(sd.flags)[FLAG_DEFERRED] : 0;
     double acc = 0.0;
-    for (int b = lane; b < n_blocks; b += 64) {
-        const int j = b - list_begin;
+    for (int b = lane; b < p.rows; b += 64) {
+        const int j = b - p.list_begin;
         if (j >= 0 && j < list_rows && (long long)j * list_per_row >= deferred) continue;
-        acc += partials[(size_t)b * len + i];
+        acc += partials[p.at(b, list_rows) * len + i];
     }
     acc = wave_sum(acc);
-    if (lane == 0) out[i] = acc;
+    if (lane == 0) out[i] = p.strings ? out[i] + acc : acc;
 }
 
 // The same sum for launches with few partial rows (at most kReduceRowsFew): one thread per element,
@@ -832,20 +846,20 @@ constexpr int kReduceRowsFew = 64;
 __global__ void __launch_bounds__(256) k_reduce_partials_few(const SlotDesc* __restrict__ slots, int n_blocks, int len,
                                                              int list_begin, int list_rows, int list_per_row) {
     const SlotDesc& sd = slots[blockIdx.z];
-    if (string_slot(sd)) return;
+    const PartialRows p(sd, n_blocks, list_begin, list_rows);
     const auto partials = to_global(sd.partials);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= len) return;
     const long long deferred = list_rows > 0 ? (long long)to_global(sd.flags)[FLAG_DEFERRED] : 0;
     double acc = 0.0;
 #pragma unroll 8
-    for (int b = 0; b < n_blocks; ++b) {
-        const int j = b - list_begin;
+    for (int b = 0; b < p.rows; ++b) {
+        const int j = b - p.list_begin;
         const bool idle = j >= 0 && j < list_rows && (long long)j * list_per_row >= deferred;
-        const double v = partials[(size_t)b * len + i];  // every row is allocated: an idle row is read, not added
+        const double v = partials[p.at(b, list_rows) * len + i];  // every row is allocated: an idle row is read, not added
         acc += idle ? 0.0 : v;
     }
-    to_global(sd.dsum)[i] = acc;
+    to_global(sd.dsum)[i] = p.strings ? to_global(sd.dsum)[i] + acc : acc;
 }
 
 // Ordered compaction of a pair list: the flagged entries of a per-entry byte array, listed in entry
@@ -863,8 +877,9 @@ struct CompactView {
     __device__ CompactView(const SlotDesc& sd, const TopoDesc& topo, int listed) {
         flag = Deferred ? sd.defer_flag : sd.singular_flag;
         out = Deferred ? sd.defer : sd.singular;
-        // the string form defers pairs only where some block may be rank deficient
-        const bool none = Deferred && string_slot(sd) && !to_global(sd.flags)[FLAG_NEAR];
+        // a string slot's flags are those of its listed pairs; where the launch has no lane kernels (listed == 0
+        // for the deferred list), no other slot has flags
+        const bool none = Deferred && (string_slot(sd) ? to_global(sd.flags)[FLAG_NEAR] == 0 : !listed);
         entries = none ? 0
                   : Deferred ? topo.n_lane_pairs
                   : listed ? (long long)to_global(sd.flags)[FLAG_DEFERRED]
@@ -2210,14 +2225,12 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
         launch_string_integrals(st, slots, z, topo);
         launch_string_forward(st, slots, z, topo);
     }
-    if (!shape.pair_kernels) {
+    if (shape.lane_fwd) {
+        if (shape.pair_kernels)
+            launch_pairs_lane(st, 0, shape.lane_blocks_fwd, slots, count, topo, shape.n_alpha, shape.n_beta,
+                              shape.lane_cond_limit);
         mark(EV_PAIR_FWD_MAIN);
-    } else if (shape.lane_fwd) {
-        if (shape.string_kernels) launch_string_defer(st, slots, z, topo);
-        launch_pairs_lane(st, 0, shape.lane_blocks_fwd, slots, count, topo, shape.n_alpha, shape.n_beta,
-                          shape.lane_cond_limit);
-        mark(EV_PAIR_FWD_MAIN);
-        compact_pairs<true>(st, slots, z, topo, 1, topo.n_lane_pairs);
+        compact_pairs<true>(st, slots, z, topo, shape.pair_kernels ? 1 : 0, topo.n_lane_pairs);
         launch_pairs_group(st, false, true, shape.list_blocks, 0, slots, count, topo, shape.mmax);
         compact_pairs<false>(st, slots, z, topo, 1, all_pairs);
     } else {
@@ -2225,7 +2238,7 @@ void launch_forward(hipStream_t st, const SlotDesc* slots, int count, const Topo
         mark(EV_PAIR_FWD_MAIN);
         compact_pairs<false>(st, slots, z, topo, 0, all_pairs);
     }
-    if (shape.pair_kernels) launch_pairs_singular(st, false, 0, slots, count, topo);
+    launch_pairs_singular(st, false, 0, slots, count, topo);
     mark(EV_PAIR_FWD);
     const long long a = (long long)topo.n_det * topo.n_str, b = (long long)topo.n_str * topo.n_str;
     hipLaunchKernelGGL(k_structure_right, dim3((unsigned)((a + 255) / 256), 1, z), dim3(256), 0, st, slots, topo);
@@ -2272,53 +2285,51 @@ void launch_backward(hipStream_t st, const SlotDesc* slots, int count, const Top
     };
     mark(EV_BWD_BEGIN);
     if (shape.string_kernels) launch_string_backward(st, slots, z, topo);
-    if (!shape.pair_kernels) {
-        for (const int k : {EV_BWD_FIELD, EV_BWD_ADJOINT, EV_BWD_KERNEL}) mark(k);
-    } else {
-        // The pair-adjoint kernels write disjoint columns (field: ds/dh; adjoint: dg) or disjoint rows
-        // (deferred list, singular pairs) of the partial rows, so for few problems the adjoint kernel and
-        // the singular-pair kernel run on the side stream beside the field and deferred-list kernels.
-        const bool fork = side && count <= kForkMaxProblems && shape.lane_bwd && !shape.string_kernels;
-        hipStream_t st2 = st;
-        if (fork) {
-            (void)hipEventRecord(side->fork, st);
-            (void)hipStreamWaitEvent(side->st, side->fork, 0);
-            st2 = side->st;
-        }
-        int part_rows = shape.pair_blocks_bwd, list_begin = 0, list_rows = 0, list_per_row = 1;
-        if (shape.lane_bwd) {
+    // The pair-adjoint kernels write disjoint columns (field: ds/dh; adjoint: dg) or disjoint rows
+    // (deferred list, singular pairs) of the partial rows, so for few problems the adjoint kernel and
+    // the singular-pair kernel run on the side stream beside the field and deferred-list kernels.
+    const bool fork = side && count <= kForkMaxProblems && shape.lane_bwd && shape.pair_kernels;
+    hipStream_t st2 = st;
+    if (fork) {
+        (void)hipEventRecord(side->fork, st);
+        (void)hipStreamWaitEvent(side->st, side->fork, 0);
+        st2 = side->st;
+    }
+    int part_rows = shape.pair_blocks_bwd, list_begin = 0, list_rows = 0, list_per_row = 1;
+    if (shape.lane_bwd) {
+        if (shape.pair_kernels)
             launch_pairs_lane(st, 1, shape.lane_blocks_bwd, slots, count, topo, shape.n_alpha, shape.n_beta,
                               shape.lane_cond_limit);
-            mark(EV_BWD_FIELD);
+        mark(EV_BWD_FIELD);
+        if (shape.pair_kernels)
             launch_pairs_lane(st2, 2, shape.lane_blocks_bwd, slots, count, topo, shape.n_alpha, shape.n_beta,
                               shape.lane_cond_limit);
-            if (!fork) mark(EV_BWD_ADJOINT);
-            list_per_row = launch_pairs_group(st, true, true, shape.list_blocks, shape.lane_blocks_bwd, slots, count, topo,
-                                              shape.mmax);
-            list_begin = shape.lane_blocks_bwd;
-            list_rows = shape.list_blocks;
-            part_rows = shape.lane_blocks_bwd + shape.list_blocks;
-        } else {
-            launch_pairs_group(st, true, false, shape.pair_blocks_bwd, 0, slots, count, topo, shape.mmax);
-            mark(EV_BWD_FIELD);
-            mark(EV_BWD_ADJOINT);
-        }
-        launch_pairs_singular(st2, true, part_rows, slots, count, topo);
-        part_rows += kSingularBlocks;
-        if (fork) {
-            (void)hipEventRecord(side->join, side->st);
-            (void)hipStreamWaitEvent(st, side->join, 0);
-            mark(EV_BWD_ADJOINT);  // field and deferred list done on the main stream, adjoint joined
-        }
-        mark(EV_BWD_KERNEL);
-        const int len = ng + 2 * n * n;
-        if (part_rows <= kReduceRowsFew)
-            hipLaunchKernelGGL(k_reduce_partials_few, dim3((len + 255) / 256, 1, z), dim3(256), 0, st, slots, part_rows,
-                               len, list_begin, list_rows, list_per_row);
-        else
-            hipLaunchKernelGGL(k_reduce_partials, dim3((len + 3) / 4, 1, z), dim3(256), 0, st, slots, part_rows, len,
-                               list_begin, list_rows, list_per_row);
+        if (!fork) mark(EV_BWD_ADJOINT);
+        list_per_row = launch_pairs_group(st, true, true, shape.list_blocks, shape.lane_blocks_bwd, slots, count, topo,
+                                          shape.mmax);
+        list_begin = shape.lane_blocks_bwd;
+        list_rows = shape.list_blocks;
+        part_rows = shape.lane_blocks_bwd + shape.list_blocks;
+    } else {
+        launch_pairs_group(st, true, false, shape.pair_blocks_bwd, 0, slots, count, topo, shape.mmax);
+        mark(EV_BWD_FIELD);
+        mark(EV_BWD_ADJOINT);
     }
+    launch_pairs_singular(st2, true, part_rows, slots, count, topo);
+    part_rows += kSingularBlocks;
+    if (fork) {
+        (void)hipEventRecord(side->join, side->st);
+        (void)hipStreamWaitEvent(st, side->join, 0);
+        mark(EV_BWD_ADJOINT);  // field and deferred list done on the main stream, adjoint joined
+    }
+    mark(EV_BWD_KERNEL);
+    const int len = ng + 2 * n * n;
+    if (part_rows <= kReduceRowsFew)
+        hipLaunchKernelGGL(k_reduce_partials_few, dim3((len + 255) / 256, 1, z), dim3(256), 0, st, slots, part_rows,
+                           len, list_begin, list_rows, list_per_row);
+    else
+        hipLaunchKernelGGL(k_reduce_partials, dim3((len + 3) / 4, 1, z), dim3(256), 0, st, slots, part_rows, len,
+                           list_begin, list_rows, list_per_row);
     mark(EV_PAIR_BWD);
     hipLaunchKernelGGL(k_ri_pair_adjoint, dim3((shape.max_n_aux + 255) / 256, (np + 7) / 8, z), dim3(256), 0, st, slots,
                        np);

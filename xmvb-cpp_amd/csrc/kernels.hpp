@@ -30,8 +30,8 @@ enum DeviceFlag : int {
     FLAG_METRIC = 3,          // structure metric not positive definite
     FLAG_DEFERRED = 4,        // pairs left by the lane kernel for the lane-group kernel (SlotDesc::defer)
     FLAG_EIGEN = 5,           // Davidson stopped without meeting its tolerances (1 + reason)
-    FLAG_STRINGS = 6,         // the slot takes the string form instead of the pair kernels
-    FLAG_NEAR = 7,            // string form: some block may be rank deficient (StringWork::neara, nearb)
+    FLAG_STRINGS = 6,         // S_act allows the string form instead of the pair kernels
+    FLAG_NEAR = 7,            // string form: pairs left to the list kernels (more than kStringListMax: pair kernels)
     FLAG_COUNT = 8
 };
 
@@ -116,9 +116,9 @@ struct LaunchShape {
     bool b32c;                             // RI factors stored as compensated FP32 (FP32 + 8-bit correction)
     bool any_tiled, any_flat;              // slots of the launch with the aux-tiled / the flat layout
     int max_n_bf_tiled;                    // largest n_bf among the slots with the aux-tiled layout
-    bool strings;                          // slots may take the string form (their FLAG_STRINGS decides)
+    bool strings;                          // slots may take the string form (string_slot decides)
     bool string_kernels;                   // launch the string form's kernels (else only the test of S_act)
-    bool pair_kernels;                     // launch the pair kernels too, for slots or pairs the string form leaves
+    bool pair_kernels;                     // launch the lane kernels too, for slots the string form leaves
     bool davidson;                         // structure eigenproblem by Davidson instead of dense
     // Pinned launch shape: every choice that changes a slot's summation order (blocks per slot of the
     // backward pair kernels, the few-problem or batched form of the Gram product, gradient tail and

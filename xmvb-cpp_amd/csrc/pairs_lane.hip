@@ -22,6 +22,7 @@
 
 #include "device.hpp"
 #include "kernels.hpp"
+#include "lane_block.hpp"
 
 namespace xmvb_amd {
 
@@ -31,95 +32,6 @@ namespace xmvb_amd {
 // the 6-electron field kernel and every adjoint kernel are slower when held to two.
 constexpr int lane_fwd_waves(int m0) { return m0 <= 6 ? 2 : 1; }
 constexpr int lane_field_waves(int m0) { return m0 <= 5 ? 2 : 1; }
-
-template <int M>
-struct LaneBlock {
-    static constexpr int K = M > 0 ? M : 1;
-    int R[K], L[K];  // occupied orbitals of the right (ket) and left (bra) strings
-    double a[K][K];  // X on entry; X^{-1} after inversion, so D[r][l] = a[l][r]
-    double det;
-};
-
-template <int M>
-__device__ __forceinline__ void occupied(uint32_t mask, int* out) {
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-        out[k] = __builtin_ctz(mask);
-        mask &= mask - 1;
-    }
-}
-
-// In-place Gauss-Jordan inversion with row pivoting. A row interchange of X is an interchange of
-// two ket orbitals, so it is applied to R as well and never undone: the result is the inverse of
-// the row-permuted block, paired with the permuted R, which every consumer sums over in any order
-// (same-spin terms are symmetric under r <-> r2; the compound W index sorts the pair itself).
-// det keeps the sign of the unpermuted block. Returns whether the block stays on the lane path.
-template <int M>
-__device__ __forceinline__ bool lane_invert(const double* __restrict__ sact, int n, double cond_limit, LaneBlock<M>& b) {
-    if constexpr (M == 0) {
-        b.det = 1.0;
-        return true;
-    } else {
-        auto& a = b.a;
-        double amax = 0.0;
-#pragma unroll
-        for (int i = 0; i < M; ++i)
-#pragma unroll
-            for (int j = 0; j < M; ++j) {
-                a[i][j] = sact[b.R[i] + n * b.L[j]];
-                amax = fmax(amax, fabs(a[i][j]));
-            }
-        double det = 1.0;
-        bool ok = true;
-#pragma unroll
-        for (int k = 0; k < M; ++k) {
-            int p = k;
-            double best = fabs(a[k][k]);
-#pragma unroll
-            for (int i = k + 1; i < M; ++i) {
-                const double v = fabs(a[i][k]);
-                const bool g = v > best;
-                best = g ? v : best;
-                p = g ? i : p;
-            }
-#pragma unroll
-            for (int i = k + 1; i < M; ++i) {
-                const bool s = p == i;
-#pragma unroll
-                for (int j = 0; j < M; ++j) {
-                    const double t = a[k][j];
-                    a[k][j] = s ? a[i][j] : t;
-                    a[i][j] = s ? t : a[i][j];
-                }
-                const int tr = b.R[k];
-                b.R[k] = s ? b.R[i] : tr;
-                b.R[i] = s ? tr : b.R[i];
-            }
-            const double pv = a[k][k];
-            ok = ok && best > 0.0;
-            det = (p != k) ? -det * pv : det * pv;
-            const double inv = best > 0.0 ? 1.0 / pv : 0.0;
-            a[k][k] = 1.0;
-#pragma unroll
-            for (int j = 0; j < M; ++j) a[k][j] *= inv;
-#pragma unroll
-            for (int i = 0; i < M; ++i) {
-                if (i == k) continue;
-                const double f = a[i][k];
-                a[i][k] = 0.0;
-#pragma unroll
-                for (int j = 0; j < M; ++j) a[i][j] -= f * a[k][j];
-            }
-        }
-        double ymax = 0.0;
-#pragma unroll
-        for (int i = 0; i < M; ++i)
-#pragma unroll
-            for (int j = 0; j < M; ++j) ymax = fmax(ymax, fabs(a[i][j]));
-        b.det = det;
-        return ok && amax * ymax < cond_limit;
-    }
-}
 
 // Same-spin two-electron energy over 2x2 minors: sum_{r<r2,l<l2} [(rl|r2l2) - (rl2|r2l)] minor.
 // pidx(r, l) is the packed pair index of block entry (R_r, L_l).

@@ -378,7 +378,6 @@ template <bool Backward, bool FullDg>
 __global__ void __launch_bounds__(256) k_pairs_singular(const SlotDesc* __restrict__ slots, TopoDesc topo,
                                                         int part_offset) {
     const SlotDesc& sd = slots[blockIdx.z];
-    if (Backward && string_slot(sd)) return;
     const int n = topo.n, ng = topo.ng, n_det = topo.n_det;
     const int np = n * (n + 1) / 2;
     const int count = to_global(sd.flags)[FLAG_SINGULAR_PAIRS];
@@ -453,7 +452,7 @@ __global__ void __launch_bounds__(256) k_pairs_singular(const SlotDesc* __restri
     if (Backward) {
         __syncthreads();
         const int stride_part = ng + 2 * n * n;
-        double* out = sd.partials + (size_t)(blockIdx.x + part_offset) * stride_part;
+        double* out = sd.partials + (size_t)(blockIdx.x + (string_slot(sd) ? kListBlocks : part_offset)) * stride_part;
         if (FullDg) {
             for (int t = threadIdx.x; t < ng; t += blockDim.x) {
                 int Q, P;

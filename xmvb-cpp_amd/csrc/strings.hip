@@ -13,16 +13,20 @@
 // sums over single replacements, where the pair kernels invert two blocks and gather 1,100 kernel
 // elements for each of 16,002 pairs.
 //
-// No overlap block is inverted, so a singular or nearly singular block costs no digits; what matters is
-// the conditioning of S_act itself, and a slot whose S_act^-1 has an element above
-// kStringInverseLimit keeps the pair kernels (FLAG_STRINGS stays clear). Every sum has a fixed order
-// that does not depend on the launch, so results are the same bits alone and in any batch.
+// No overlap block is inverted; what matters is the conditioning of S_act itself, and a slot whose S_act^-1
+// has an element above kStringInverseLimit keeps the pair kernels (FLAG_STRINGS stays clear). Pairs whose
+// regular inverse form loses digits, and those it does not cover, stay with the list kernels
+// (k_pairs, k_pairs_singular) in the energy and the gradient, as they do behind the lane kernels: the
+// results are those of the pair kernels to their own rounding (kStringListError), whichever form a launch takes.
+// Every sum here has a fixed order that does not depend on the launch; the list kernels' rows follow the
+// batch unless the launch is pinned.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
 #include "device.hpp"
 #include "kernels.hpp"
+#include "lane_block.hpp"
 #include "wave.hpp"
 
 namespace xmvb_amd {
@@ -110,13 +114,11 @@ __global__ void __launch_bounds__(256) k_string_minors(const SlotDesc* __restric
         }
     }
     const auto out = to_global(beta ? sd.sw.Mb : sd.sw.Ma);
-    const auto near = to_global(beta ? sd.sw.nearb : sd.sw.neara);
-    bool any_near = false;
     for (int u = 0; u < kMinorRows; ++u) {
         const int x = blockIdx.y * kMinorRows + u;
         if (x >= sp.N) break;
         uint32_t rows = sp.mask[x];
-        double D[1 << M], norm2 = 0.0;
+        double D[1 << M];
         D[0] = 1.0;
 #pragma unroll
         for (int k = 1; k <= M; ++k) {
@@ -124,10 +126,7 @@ __global__ void __launch_bounds__(256) k_string_minors(const SlotDesc* __restric
             rows &= rows - 1;
             double v[M];
 #pragma unroll
-            for (int j = 0; j < M; ++j) {
-                v[j] = row[L[j]];
-                norm2 += v[j] * v[j];
-            }
+            for (int j = 0; j < M; ++j) v[j] = row[L[j]];
 #pragma unroll
             for (int c = 1; c < (1 << M); ++c) {
                 if (__builtin_popcount(c) != k) continue;
@@ -143,19 +142,61 @@ __global__ void __launch_bounds__(256) k_string_minors(const SlotDesc* __restric
                 D[c] = acc;
             }
         }
-        const double det = D[(1 << M) - 1];
-        out[(size_t)x * sp.N + y] = det;
-        // sigma_min >= |det| ((M - 1) / |X|_F^2)^((M - 1) / 2); a NaN counts as near
-        const double ratio = (M - 1) / norm2;
-        double bound = fabs(det);
-#pragma unroll
-        for (int k = 0; k < (M - 1) / 2; ++k) bound *= ratio;
-        if (M > 1 && M % 2 == 0) bound *= sqrt(ratio);
-        const bool is_near = !(bound > kStringRegularSigma);
-        near[(size_t)x * sp.N + y] = is_near ? 1 : 0;
-        any_near = any_near || is_near;
+        out[(size_t)x * sp.N + y] = D[(1 << M) - 1];
     }
-    if (any_near) to_global(sd.flags)[FLAG_NEAR] = 1;
+}
+
+// Conditioning of the overlap block of every string pair: 0 where the lane kernels keep it, else the power of
+// two above max|X^-1|, or kMaybeSingular where the complete-pivoting rank rule may call it deficient. One
+// unordered pair per lane, inverted in registers as the lane kernels do. FP64 VALU bound.
+constexpr int kMaybeSingular = 255;
+template <int M>
+__global__ void __launch_bounds__(256) k_string_condition(const SlotDesc* __restrict__ slots, int n, StringSpace sp,
+                                                          bool beta) {
+    const SlotDesc& sd = slots[blockIdx.z];
+    if (!to_global(sd.flags)[FLAG_STRINGS]) return;
+    __shared__ double s[kMaxN * kMaxN];
+    for (int t = threadIdx.x; t < n * n; t += blockDim.x) s[t] = to_global(sd.sact)[t];
+    __syncthreads();
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)sp.N * (sp.N + 1) / 2) return;
+    int x, y;
+    unpack_pair(t, x, y);
+    LaneBlock<M> b;
+    occupied<M>(sp.mask[x], b.R);
+    occupied<M>(sp.mask[y], b.L);
+    int code = 0;
+    if (!lane_invert<M>(s, n, kLaneConditionDefault, b))  // a NaN counts as singular
+        code = b.cond < kLaneConditionMax ? ilogb(b.inverse) + 1 : kMaybeSingular;
+    const auto near = to_global(beta ? sd.sw.nearb : sd.sw.neara);
+    near[(size_t)x * sp.N + y] = (unsigned char)code;
+    near[(size_t)y * sp.N + x] = (unsigned char)code;
+}
+
+// Pairs left to the list kernels (kStringListError), flagged per work item of the lane kernels, so that
+// they are listed as the lane kernels' own deferred pairs are, and counted in FLAG_NEAR.
+__global__ void __launch_bounds__(256) k_string_list(const SlotDesc* __restrict__ slots, TopoDesc topo) {
+    const SlotDesc& sd = slots[blockIdx.z];
+    if (!to_global(sd.flags)[FLAG_STRINGS]) return;
+    const StringTopo& t = topo.str;
+    const int na = t.a.N, nb = t.b.N;
+    const auto pa = to_global(sd.sw.neara), pb = to_global(sd.sw.nearb);
+    const double limit = kStringListError * topo.n_det;
+    int count = 0;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < topo.n_lane_pairs;
+         i += (long long)gridDim.x * blockDim.x) {
+        int d, e;
+        unpack_pair(topo.lane_pairs ? (long long)topo.lane_pairs[i] : i, d, e);
+        const size_t a = (size_t)t.arank[d] * na + t.arank[e], b = (size_t)t.brank[d] * nb + t.brank[e];
+        const int p = max((int)pa[a], (int)pb[b]);
+        const bool listed =
+            p == kMaybeSingular || (p > 0 && ldexp(fabs(to_global(sd.sw.Ma)[a] * to_global(sd.sw.Mb)[b]), 3 * p) >= limit);
+        to_global(sd.defer_flag)[i] = listed;
+        count += listed ? (topo.flip ? 2 : 1) : 0;
+    }
+#pragma unroll
+    for (int off = 32; off; off >>= 1) count += __shfl_xor(count, off, 64);
+    if ((threadIdx.x & 63) == 0 && count) atomicAdd(sd.flags + FLAG_NEAR, count);
 }
 
 // ---- transformed integrals --------------------------------------------------------------------------
@@ -537,22 +578,6 @@ __global__ void __launch_bounds__(256) k_string_pairs(const SlotDesc* __restrict
     }
 }
 
-// Pairs with a block that may be rank deficient: flagged per work item of the lane kernels, so that
-// they are listed and evaluated by the complete-pivoting kernel as the lane kernels' own deferred
-// pairs are. Slots without such a block (FLAG_NEAR clear) have nothing to list.
-__global__ void __launch_bounds__(256) k_string_defer(const SlotDesc* __restrict__ slots, TopoDesc topo) {
-    const SlotDesc& sd = slots[blockIdx.z];
-    if (!string_slot(sd) || !to_global(sd.flags)[FLAG_NEAR]) return;
-    const StringTopo& t = topo.str;
-    const auto pa = to_global(sd.sw.neara), pb = to_global(sd.sw.nearb);
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < topo.n_lane_pairs;
-         i += (long long)gridDim.x * blockDim.x) {
-        int d, e;
-        unpack_pair(topo.lane_pairs ? (long long)topo.lane_pairs[i] : i, d, e);
-        to_global(sd.defer_flag)[i] = pa[(size_t)t.arank[d] * t.a.N + t.arank[e]] | pb[(size_t)t.brank[d] * t.b.N + t.brank[e]];
-    }
-}
-
 // f = M_a (C M_b)
 template <bool Few>
 __global__ void __launch_bounds__(256) k_string_bra(const SlotDesc* __restrict__ slots, TopoDesc topo, int tiles,
@@ -829,6 +854,33 @@ __global__ void __launch_bounds__(256) k_string_same(const SlotDesc* __restrict_
 // f and sigma operands have the same index, so one table entry and one 16-byte LDS read serve both; R rows
 // share the table read. Bound by those LDS reads (gathers). One thread per (q, l) over lists of
 // strings took 288 us for 192 problems of 10 orbitals and 1.77 ms for one of 14.
+template <int R, typename P>
+__device__ __forceinline__ void response_products(const f64x2* rows, P wtab, int nb, int nw, string_double4& acc) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+#pragma unroll 4
+    for (int w0 = 4 * wave; w0 < nw; w0 += 16) {
+        const int w = w0 + k4;
+        const uint32_t code = wtab[(size_t)min(w, nw - 1) * 16 + i16];
+        const int at = w < nw ? (int)(code & 0xfff) : nb;
+        const uint32_t odd = code << 16;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const f64x2 v = rows[r * (nb + 1) + at];
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(signed_value(v[0], odd), signed_value(v[1], odd), acc, 0, 0, 0);
+        }
+    }
+}
+
+// Element (q, l) = (threadIdx.x / 16, threadIdx.x % 16) of the four wavefronts' sums; lds: 4 x 256
+__device__ __forceinline__ double response_sum(double* lds, const string_double4& acc) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) lds[wave * 256 + (4 * v + k4) * 16 + i16] = acc[v];
+    __syncthreads();
+    return (lds[threadIdx.x] + lds[256 + threadIdx.x]) + (lds[512 + threadIdx.x] + lds[768 + threadIdx.x]);
+}
+
 template <int R>
 __global__ void __launch_bounds__(256) k_string_response(const SlotDesc* __restrict__ slots, TopoDesc topo,
                                                          int accumulate) {
@@ -838,11 +890,10 @@ __global__ void __launch_bounds__(256) k_string_response(const SlotDesc* __restr
     if (!string_slot(sd)) return;
     extern __shared__ double lds[];
     const StringTopo& t = topo.str;
-    const int n = topo.n, na = t.a.N, nb = t.b.N, nw = t.nw;
+    const int n = topo.n, na = t.a.N, nb = t.b.N;
     f64x2* rows = reinterpret_cast<f64x2*>(lds);  // [R][nb + 1]: (f, sigma), zeros at nb
     const auto f = to_global(static_cast<const double*>(sd.Hdet));
     const auto sg = to_global(static_cast<const double*>(sd.Sdet));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
     string_double4 acc = string_double4{0.0, 0.0, 0.0, 0.0};
     const int last = min(na, (bx + 1) * kStringRowsZ);
     for (int x = bx * kStringRowsZ; x < last; x += R) {
@@ -854,26 +905,11 @@ __global__ void __launch_bounds__(256) k_string_response(const SlotDesc* __restr
                 rows[r * (nb + 1) + i] = live ? f64x2{f[at], sg[at]} : f64x2{0.0, 0.0};
             }
         __syncthreads();
-#pragma unroll 4
-        for (int w0 = 4 * wave; w0 < nw; w0 += 16) {
-            const int w = w0 + k4;
-            const uint32_t code = t.wtab[(size_t)min(w, nw - 1) * 16 + i16];
-            const int at = w < nw ? (int)(code & 0xfff) : nb;
-            const uint32_t odd = code << 16;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const f64x2 v = rows[r * (nb + 1) + at];
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(signed_value(v[0], odd), signed_value(v[1], odd), acc, 0, 0, 0);
-            }
-        }
+        response_products<R>(rows, t.wtab, nb, t.nw, acc);
     }
-    __syncthreads();
-#pragma unroll
-    for (int v = 0; v < 4; ++v) lds[wave * 256 + (4 * v + k4) * 16 + i16] = acc[v];
-    __syncthreads();
+    const double s = response_sum(lds, acc);
     const int q = threadIdx.x >> 4, l = threadIdx.x & 15;
     if (q < n && l < n) {
-        const double s = (lds[threadIdx.x] + lds[256 + threadIdx.x]) + (lds[512 + threadIdx.x] + lds[768 + threadIdx.x]);
         const auto out = to_global(sd.sw.zpart) + (size_t)bx * n * n + q * n + l;
         *out = accumulate ? *out + s : s;
     }
@@ -907,9 +943,171 @@ __global__ void __launch_bounds__(256) k_string_response_alpha(const SlotDesc* _
     }
 }
 
+// ---- listed pairs ------------------------------------------------------------------------------------------
+
+// The densities above sum over all pairs; those of the listed ones, which the list kernels differentiate, are
+// taken out again as one more chunk. One wavefront per (q, l) (opposite spin), then per (l < l2) of each
+// spin (beta alone under spin-exchange symmetry), over the listed pairs in order, each pair both ways
+// (d ket, e bra); lanes over the ket's replacements. Bound by the chain of dependent reads of a pair, about 1 us.
+__global__ void __launch_bounds__(256) k_string_list_density(const SlotDesc* __restrict__ slots, TopoDesc topo) {
+    const SlotDesc& sd = slots[blockIdx.z];
+    if (!string_slot(sd)) return;
+    __shared__ double lds[4][kMaxN * kMaxN];
+    const StringTopo& t = topo.str;
+    const int n = topo.n, n2 = n * n, nc = n * (n - 1) / 2, na = t.a.N, nb = t.b.N;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int item = blockIdx.x * 4 + wave;
+    if (item >= n2 + (t.sym ? 1 : 2) * nc) return;
+    const bool opposite = item < n2, alpha = item >= n2 + nc;
+    const int L = item - n2 - (alpha ? nc : 0);
+    int x = item / n, y = item - x * n;  // opposite spin: y -> x of the alpha string; same spin: the two replaced
+    if (!opposite) {
+        unpack_pair(L, x, y);
+        ++y;
+    }
+    double* acc = lds[wave];
+    const int len = opposite ? n2 : nc;
+    for (int i = lane; i < len; i += 64) acc[i] = 0.0;
+    wave_sync();
+    const auto Ma = to_global(static_cast<const double*>(sd.sw.Ma)), Mb = to_global(static_cast<const double*>(sd.sw.Mb));
+    const StringSpace& own = opposite || alpha ? t.a : t.b;  // the string that the wavefront's item selects
+    const int listed = to_global(sd.flags)[FLAG_DEFERRED];
+    for (int i = 0; i < listed; ++i) {
+        int d, e;
+        unpack_pair(to_global(sd.defer)[i], d, e);
+        double w, unused;
+        pair_weights(sd, topo, d, e, d, e, false, 1.0, w, unused);
+        for (int way = 0; way < (d == e ? 1 : 2); ++way) {
+            const int bra = way ? e : d, ket = way ? d : e;
+            const int a = t.arank[ket], b = t.brank[ket], A = t.arank[bra], B = t.brank[bra];
+            const uint32_t mask = own.mask[opposite || alpha ? a : b];
+            if (opposite) {
+                if (!(mask >> y & 1) || (x != y && (mask >> x & 1))) continue;
+                const uint32_t left = mask ^ (1u << y);
+                const double m = Ma[(size_t)A * na + t.rank[left | 1u << x]];
+                const double u = -w * ((below(mask, y) + below(left, x)) & 1 ? -m : m);
+                if (lane < t.b.J) {
+                    const uint32_t code = t.b.e1[(size_t)b * t.b.J + lane];
+                    acc[code >> 16 & 0xff] += signed_value(u * Mb[(size_t)B * nb + (code & 0xffff)], code);
+                }
+            } else {
+                if (!(mask >> x & 1) || !(mask >> y & 1)) continue;
+                const int k1 = below(mask, x), k2 = below(mask, y), pairs = own.m * (own.m - 1) / 2;
+                const int nq = alpha ? t.nq_a : t.nq_b;
+                const uint32_t* list = (alpha ? t.e2a : t.e2b) + ((size_t)(alpha ? a : b) * pairs + k2 * (k2 - 1) / 2 + k1) * nq;
+                const auto M = alpha ? Ma + (size_t)A * na : Mb + (size_t)B * nb;
+                const double u = -w * (alpha ? Mb[(size_t)B * nb + b] : Ma[(size_t)A * na + a]);
+                for (int q = lane; q < nq; q += 64) acc[list[q] >> 12 & 0x7f] += signed_value(u * M[list[q] & 0xfff], list[q]);
+            }
+        }
+    }
+    wave_sync();
+    const auto out = opposite ? to_global(sd.sw.gpart) + ((size_t)t.gchunks * n2 + item) * n2
+                              : to_global(sd.sw.wpart) + ((size_t)((t.sym ? 1 : 2) * t.wchunks + (alpha ? 1 : 0)) * nc + L) * nc;
+    for (int i = lane; i < len; i += 64) out[i] = acc[i];
+}
+
+// The listed pairs' response, rows zblocks.. of zpart: workgroup k takes pairs k, k + kStringListRows, ...
+// Both rows of a pair are products of one vector per spin: f = M_a[d_a] M_b[d_b], and sigma = (Ht - E) e is
+// contracted with the other spin's row of M, so that the beta part is the response of the strings
+//   (M_b[d_b][y], t[y]),  t[y] = sum_x M_a[d_a][x] sigma[x][y]
+// as one more row of k_string_response, and the alpha part (without spin-exchange symmetry) its mirror image.
+__global__ void __launch_bounds__(256) k_string_list_response(const SlotDesc* __restrict__ slots, TopoDesc topo,
+                                                              int zblocks) {
+    const SlotDesc& sd = slots[blockIdx.z];
+    if (!string_slot(sd)) return;
+    extern __shared__ __align__(16) double lds[];
+    __shared__ double ua[64], ub[64], part[2][4];
+    const StringTopo& t = topo.str;
+    const int n = topo.n, n2 = n * n, na = t.a.N, nb = t.b.N, Ja = t.a.J, Jb = t.b.J, tid = threadIdx.x;
+    f64x2* rows = reinterpret_cast<f64x2*>(lds);  // (M_b[d_b][y], t[y]), zeros at nb
+    double* ta = lds + 2 * (nb + 1);
+    const auto Ma = to_global(static_cast<const double*>(sd.sw.Ma)), Mb = to_global(static_cast<const double*>(sd.sw.Mb));
+    const auto Ha = to_global(static_cast<const double*>(sd.sw.Ha)), Hb = to_global(static_cast<const double*>(sd.sw.Hb));
+    const auto gt = to_global(static_cast<const double*>(sd.sw.gt));
+    string_double4 acc = string_double4{0.0, 0.0, 0.0, 0.0};
+    double alpha = 0.0;  // element tid of the alpha part
+    const int listed = to_global(sd.flags)[FLAG_DEFERRED];
+    for (int i = blockIdx.x; i < listed; i += gridDim.x) {
+        int d, e;
+        unpack_pair(to_global(sd.defer)[i], d, e);
+        double wH, wS;
+        pair_weights(sd, topo, d, e, d, e, false, 1.0, wH, wS);
+        for (int way = 0; way < (d == e ? 1 : 2); ++way) {
+            const int bra = way ? e : d, ket = way ? d : e;
+            const int a = t.arank[ket], b = t.brank[ket], A = t.arank[bra], B = t.brank[bra];
+            const uint32_t* ea = t.a.e1 + (size_t)a * Ja;
+            const uint32_t* eb = t.b.e1 + (size_t)b * Jb;
+            const double ma = Ma[(size_t)A * na + a], mb = Mb[(size_t)B * nb + b];
+            __syncthreads();  // the previous pair's rows have been read
+            if (tid < Ja) ua[tid] = signed_value(Ma[(size_t)A * na + (ea[tid] & 0xffff)], ea[tid]);
+            if (tid >= 64 && tid < 64 + Jb) ub[tid - 64] = signed_value(Mb[(size_t)B * nb + (eb[tid - 64] & 0xffff)], eb[tid - 64]);
+            // K = M Ht of the pair, either spin
+            double ka = 0.0, kb = 0.0;
+            for (int x = tid; x < na; x += 256) ka += Ma[(size_t)A * na + x] * Ha[(size_t)x * na + a];
+            for (int y = tid; y <= nb; y += 256) {
+                const double m = y < nb ? Mb[(size_t)B * nb + y] : 0.0, h = y < nb ? Hb[(size_t)y * nb + b] : 0.0;
+                kb += m * h;
+                rows[y] = f64x2{m, wH * ma * h};
+            }
+            if (!t.sym)
+                for (int x = tid; x < na; x += 256) ta[x] = wH * mb * Ha[(size_t)x * na + a];
+            ka = wave_sum(ka);
+            kb = wave_sum(kb);
+            if ((tid & 63) == 0) {
+                part[0][tid >> 6] = ka;
+                part[1][tid >> 6] = kb;
+            }
+            __syncthreads();
+            // opposite spin: wavefront 0 adds the beta targets, 1 the alpha ones (distinct but for the string itself)
+            const bool beta = tid < 64;
+            if (beta || (tid < 128 && !t.sym)) {
+                const int j = tid & 63, J = beta ? Jb : Ja, J2 = beta ? Ja : Jb, noff = beta ? t.b.noff : t.a.noff;
+                double v = 0.0;
+                const uint32_t code = beta ? eb[min(j, J - 1)] : ea[min(j, J - 1)];
+                const int own = (int)(code >> 16 & 0xff);
+#pragma unroll 4
+                for (int k = 0; k < J2; ++k) {
+                    const int other = (int)((beta ? ea[k] : eb[k]) >> 16 & 0xff);
+                    v += (beta ? ua[k] : ub[k]) * gt[beta ? other * n2 + own : own * n2 + other];
+                }
+                v = signed_value(wH * v, code);
+                const double itself = wave_sum(j >= noff && j < J ? v : 0.0);
+                if (j < noff) {
+                    if (beta) rows[code & 0xffff][1] += v;
+                    else ta[code & 0xffff] += v;
+                }
+                if (j == 0) {
+                    const double* p = part[beta ? 0 : 1];
+                    const double k = (p[0] + p[1]) + (p[2] + p[3]);
+                    const double s = itself + wH * k + wS * (beta ? ma : mb);
+                    if (beta) rows[b][1] += s;
+                    else ta[a] += s;
+                }
+            }
+            __syncthreads();
+            response_products<1>(rows, t.wtab, nb, t.nw, acc);
+            if (!t.sym && tid < n2) {
+                for (int k = 0; k < t.ak; ++k) {
+                    const uint32_t at = t.alist[(size_t)k * n2 + tid];
+                    if (at == ~0u) continue;
+                    const uint32_t code = t.a.e1[at];
+                    alpha += signed_value(Ma[(size_t)A * na + (code & 0xffff)] * ta[at / Ja], code);
+                }
+            }
+        }
+    }
+    const double s = response_sum(lds, acc);
+    __syncthreads();
+    lds[tid] = alpha;
+    __syncthreads();
+    const int q = tid >> 4, l = tid & 15;
+    if (q < n && l < n) to_global(sd.sw.zpart)[(size_t)(zblocks + blockIdx.x) * n2 + q * n + l] = -(s + lds[q * n + l]);
+}
+
 // ---- adjoints ------------------------------------------------------------------------------------------
 
-// gs = dgt + dgt^T from the chunks of the densities: a workgroup takes the 16 x 16 tiles (X, Y) and (Y, X), both
+// gs = dgt + dgt^T from the chunks of the densities, the listed pairs' last: a workgroup takes the 16 x 16 tiles (X, Y) and (Y, X), both
 // read along their rows and exchanged through LDS. The last workgroup forms dht and Z.
 constexpr int kGatherTile = 16;
 __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restrict__ slots, TopoDesc topo, int tiles,
@@ -932,7 +1130,7 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
         double v = 0.0, v2 = 0.0;
         const size_t at = (size_t)min(X, n2 - 1) * n2 + min(Y, n2 - 1), at2 = (size_t)min(X2, n2 - 1) * n2 + min(Y2, n2 - 1);
 #pragma unroll 4
-        for (int k = 0; k < t.gchunks; ++k) {
+        for (int k = 0; k <= t.gchunks; ++k) {
             v += gp[k * n4 + at];
             v2 += gp[k * n4 + at2];
         }
@@ -948,7 +1146,7 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
             const auto w = to_global(static_cast<const double*>(sd.sw.wpart)) + (size_t)(lb * (lb - 1) / 2 + la) * nc +
                            qb * (qb - 1) / 2 + qa;
             double s = 0.0;
-            for (int k = 0; k < (t.sym ? t.wchunks : 2 * t.wchunks); ++k) s += w[(size_t)k * nc * nc];
+            for (int k = 0; k < (t.sym ? 1 : 2) * (t.wchunks + 1); ++k) s += w[(size_t)k * nc * nc];
             if (t.sym) s *= 2.0;
             return (q < q2) == (l < l2) ? s : -s;
         };
@@ -960,7 +1158,7 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
     // dht over both spins: a diagonal of the density counts every electron of the other spin
     for (int X = threadIdx.x; X < n2; X += 256) {
         double va = 0.0, vb = 0.0;
-        for (int k = 0; k < t.gchunks; ++k)
+        for (int k = 0; k <= t.gchunks; ++k)
             for (int l = 0; l < n; ++l) {
                 va += gp[k * n4 + (size_t)X * n2 + l * (n + 1)];
                 vb += gp[k * n4 + (size_t)l * (n + 1) * n2 + X];
@@ -1050,10 +1248,12 @@ int z_blocks(const StringTopo& t) { return (t.a.N + kStringRowsZ - 1) / kStringR
 template <int M>
 void minors(hipStream_t st, const SlotDesc* slots, unsigned z, int n, const StringSpace& sp, bool beta) {
     if constexpr (M > 8) return;
-    else if (sp.m == M)
+    else if (sp.m == M) {
         hipLaunchKernelGGL(k_string_minors<M>, dim3(blocks_for(sp.N), (unsigned)((sp.N + kMinorRows - 1) / kMinorRows), z),
                            dim3(256), 0, st, slots, n, sp, beta);
-    else minors<M + 1>(st, slots, z, n, sp, beta);
+        hipLaunchKernelGGL(k_string_condition<M>, dim3(blocks_for((long long)sp.N * (sp.N + 1) / 2), 1, z), dim3(256), 0, st,
+                           slots, n, sp, beta);
+    } else minors<M + 1>(st, slots, z, n, sp, beta);
 }
 
 }  // namespace
@@ -1094,9 +1294,9 @@ size_t string_work_carve(const TopoDesc& topo, double* base, StringWork& w) {
     else take(w.Kb, nb * nb);
     const size_t after_k = at;
     at = shared;
-    take(w.gpart, (size_t)t.gchunks * n4);
-    take(w.wpart, (size_t)t.wchunks * (t.sym ? 1 : 2) * nc * nc);
-    take(w.zpart, (size_t)z_blocks(t) * n2 + na * t.a.J);
+    take(w.gpart, (size_t)(t.gchunks + 1) * n4);
+    take(w.wpart, (size_t)(t.wchunks + 1) * (t.sym ? 1 : 2) * nc * nc);
+    take(w.zpart, (size_t)(z_blocks(t) + kStringListRows) * n2 + na * t.a.J);
     take(w.gs, n4);
     take(w.hb, n2);
     take(w.V, n4);
@@ -1113,6 +1313,8 @@ void launch_string_minors(hipStream_t st, const SlotDesc* slots, unsigned z, con
     const StringTopo& t = topo.str;
     minors<1>(st, slots, z, topo.n, t.a, false);
     if (t.a.m != t.b.m) minors<1>(st, slots, z, topo.n, t.b, true);
+    hipLaunchKernelGGL(k_string_list, dim3((unsigned)std::min<long long>(256, (topo.n_lane_pairs + 255) / 256), 1, z),
+                       dim3(256), 0, st, slots, topo);
 }
 
 void launch_string_integrals(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo) {
@@ -1157,15 +1359,10 @@ void launch_string_forward(hipStream_t st, const SlotDesc* slots, unsigned z, co
     string_pairs<2>(st, slots, z, topo, (std::max(t.a.noff, t.b.noff) + 4) / 4);
 }
 
-void launch_string_defer(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo) {
-    hipLaunchKernelGGL(k_string_defer, dim3((unsigned)std::min<long long>(64, (topo.n_lane_pairs + 255) / 256), 1, z),
-                       dim3(256), 0, st, slots, topo);
-}
-
 void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo) {
     const StringTopo& t = topo.str;
     const int n = topo.n, n2 = n * n, nc = n * (n - 1) / 2, na = t.a.N, nb = t.b.N;
-    const int wc = t.wchunks, zb = z_blocks(t);
+    const int wc = t.wchunks, zb = z_blocks(t), zrows = zb + kStringListRows;
     const dim3 w_grid((unsigned)((nc * wc + 3) / 4), 1, z);
     const int ti = (na + kProductTile - 1) / kProductTile, tj = (nb + kProductTile - 1) / kProductTile;
     const int row_waves = nb > 1000 ? 2 : 4;  // two wavefronts' rows of 3432 strings leave two workgroups per CU
@@ -1198,12 +1395,16 @@ void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, c
         if (!t.sym) {
             if (wc > 0) hipLaunchKernelGGL(k_string_same<true>, w_grid, dim3(256), 0, st, slots, topo, s, wc, add);
             hipLaunchKernelGGL(k_string_response_alpha, dim3((unsigned)na, 1, z), dim3(256), sizeof(double) * nb, st, slots,
-                               topo, zb * n2, add);
+                               topo, zrows * n2, add);
         }
     }
+    hipLaunchKernelGGL(k_string_list_density, dim3((unsigned)((n2 + (t.sym ? 1 : 2) * nc + 3) / 4), 1, z), dim3(256), 0, st,
+                       slots, topo);
+    hipLaunchKernelGGL(k_string_list_response, dim3(kStringListRows, 1, z), dim3(256),
+                       sizeof(double) * std::max<size_t>(2 * (nb + 1) + (t.sym ? 0 : na), 4 * 256), st, slots, topo, zb);
     const long long n4 = (long long)n2 * n2;
     const int gt = (n2 + kGatherTile - 1) / kGatherTile, gtiles = gt * (gt + 1) / 2;
-    hipLaunchKernelGGL(k_string_gather, dim3((unsigned)gtiles + 1, 1, z), dim3(256), 0, st, slots, topo, gtiles, zb);
+    hipLaunchKernelGGL(k_string_gather, dim3((unsigned)gtiles + 1, 1, z), dim3(256), 0, st, slots, topo, gtiles, zrows);
     const unsigned vb = blocks_for(n4);
     hipLaunchKernelGGL(k_string_pullback, dim3(vb + n2, 1, z), dim3(256), 0, st, slots, n, (int)vb);
     hipLaunchKernelGGL(k_string_adjoint, dim3(blocks_for(topo.ng + 2 * n2), 1, z), dim3(256), 0, st, slots, n, topo.ng);
@@ -1213,8 +1414,9 @@ hipError_t configure_strings() {
     for (const void* k : {reinterpret_cast<const void*>(&k_string_sigma),
                           reinterpret_cast<const void*>(&k_string_response<1>),
                           reinterpret_cast<const void*>(&k_string_response<2>),
-                          reinterpret_cast<const void*>(&k_string_response<4>)}) {
-        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+                          reinterpret_cast<const void*>(&k_string_response<4>),
+                          reinterpret_cast<const void*>(&k_string_list_response)}) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -105,7 +105,7 @@ struct StringWork {
     double *Ma, *Mb;     // minors of S_act over all string pairs
     double *Ja, *Jb;     // sum over the occupied l2 of gt[q n + l][l2 l2], per string
     double *Ha, *Hb;     // same-spin Hamiltonian in the dual frame, [x][a]
-    unsigned char *neara, *nearb;  // string pairs whose overlap block may be rank deficient
+    unsigned char *neara, *nearb;  // string pairs: conditioning of the overlap block (k_string_condition)
     double *Ka, *Kb;     // same-spin Hamiltonian between strings; during the forward, over gpart and on
     double *gpart, *wpart, *zpart;
     double *gs, *hb, *V, *W2, *Zt;
@@ -119,10 +119,18 @@ struct StringWork {
 constexpr int kStringDets = 200, kStringDetsBatched = 100, kStringBatch = 16;
 constexpr int kStringRowsZ = 8;         // rows of f and sigma per workgroup of the response sum
 constexpr int kStringPairSegment = 128; // determinants per wavefront of k_string_pairs (512 in large spaces)
-// A block whose smallest singular value is provably above this is regular under the complete-pivoting rank
-// rule: its pivots are at least sigma_min / m and at most 16 max|X| <= 16, a ratio above 7e-12 for m <= 8
-// against the rule's 1e-12, and no singular value is below the rule's absolute 1e-12.
-constexpr double kStringRegularSigma = 1.0e-9;
+// Pairs left to the list kernels, energy and gradient: those whose regular inverse form loses digits, so that
+// both forms give the same result whatever the slot, the batch or the limits choose. The inverse form of the
+// gradient cancels terms of size |S_de| max|X^-1|^3 down to S_de's own size. Over 1,477 problems of 9 to 14 orbitals
+// the relative difference of the two forms' gradients stayed below 1e-17 times the sum of that over the pairs of
+// the strings, divided by the number of determinants (median 8e-20), and reached 8.8e-6 without a list. This
+// limit per pair (divided likewise) keeps the sum below 7e6; the difference then stayed below 1.8e-10, with a median
+// of 2 pairs listed at 10 orbitals and 20 at 12 to 14. A block the lane kernels keep (condition below
+// kLaneConditionDefault) is never listed; one that may be rank deficient (above kLaneConditionMax) always is.
+constexpr double kStringListError = 1.0e5;
+// Above this many listed pairs a slot stays on the pair kernels: the list costs about 1 us a pair.
+constexpr int kStringListMax = 256;
+constexpr int kStringListRows = 32;     // workgroups (partial rows) of the listed pairs' response
 // Largest |S_act^-1| element (orbitals of unit norm) for which a slot takes the string form.
 constexpr double kStringInverseLimit = 16.0;
 
@@ -134,15 +142,13 @@ std::size_t string_work_carve(const TopoDesc& topo, double* base, StringWork& w)
 
 // S_act^-1 and the route of each slot (FLAG_STRINGS); after the active matrices
 void launch_string_frame(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
-// minors of S_act and the blocks that may be rank deficient
+// minors of S_act and the pairs left to the list kernels (flags per work item of the lane kernels, FLAG_NEAR)
 void launch_string_minors(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
 // transformed integrals and the same-spin Hamiltonian
 void launch_string_integrals(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
 // determinant matrices (SlotDesc::Hdet, Sdet)
 void launch_string_forward(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
-// flags of the pairs with a block that may be rank deficient, left to the lane-group kernel
-void launch_string_defer(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
-// adjoints of the packed kernel, S_act and h_act into SlotDesc::dsum
+// adjoints of the packed kernel, S_act and h_act into SlotDesc::dsum, without the listed pairs
 void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo);
 hipError_t configure_strings();
 
