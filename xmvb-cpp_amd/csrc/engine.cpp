@@ -711,6 +711,12 @@ void load_slot(vbe_pool* p, int slot, int n_bf, int n_aux, const double* S, cons
     s.loaded = true;
 }
 
+// kStringWork's measure of a launch of `count` problems
+double string_work(const vbe_pool* p, long long count) {
+    const double pair = (double)p->topo.n_det * p->n_alpha * p->n_beta;
+    return pair * pair * (double)count;
+}
+
 // Per-slot inputs of one launch.
 struct SlotInput {
     int slot;
@@ -766,7 +772,7 @@ LaunchShape shape_for(const vbe_pool* p, const std::vector<SlotInput>& in, bool 
     // with another program, or force their complete-pivoting path); the default leaves the choice
     // to each slot's S_act.
     sh.strings = p->topo.str.enabled && sh.lane_bwd && sh.lane_cond_limit == xmvb_amd::kLaneConditionDefault &&
-                 (p->topo.n_det >= xmvb_amd::kStringDets || (!pinned && count >= xmvb_amd::kStringBatch));
+                 string_work(p, pinned ? 1 : count) >= xmvb_amd::kStringWork;
     for (const auto& x : in) sh.strings = sh.strings && p->slots[x.slot].desc.sw.Sinv;
     sh.davidson = p->eigensolver == VBE_EIGENSOLVER_DAVIDSON;
     if (sh.davidson && (p->topo.n_states > 1 || p->topo.state_idx[0] != 0))

@@ -112,11 +112,16 @@ struct StringWork {
     double *Fa, *Fb;     // ht + Coulomb - exchange of each string, [x][ql]
 };
 
-// Where the string form is the faster one (both measured in one build, in us, string form / pair kernels):
-// one problem of 70, 126, 252, 462 determinants 372/345, 528/460, 515/506, 2326/2718; 32 problems
-// 402/389, 651/749, 747/1469, 4446/12988. So always from kStringDets on, and from kStringDetsBatched for
-// launches of at least kStringBatch problems (never for pinned shapes, whose form may not depend on the batch).
-constexpr int kStringDets = 200, kStringDetsBatched = 100, kStringBatch = 16;
+// Where the string form is the faster one: from kStringWork on of the pair kernels' leading work, n_det^2 (m_a m_b)^2
+// over all problems of the launch (of one problem for pinned shapes, whose form may not depend on the batch).
+// Both forms in one build, whole calls of 100 basis functions in us, string form / pair kernels, by that work: 126 determinants
+// (5 + 4 electrons) x 16 1.0e8 837/702, x 64 4.1e8 1501/1607; 210 (6 + 4) x 1 2.5e7 1137/903, x 8 2.0e8 1284/1364; 252
+// (5 + 5) x 1 4.0e7 540/518, x 4 1.6e8 676/628, x 8 3.2e8 721/783, x 64 2.5e9 1740/2700; 400 on 20 strings (3 + 3) x 8
+// 1.0e8 1393/1317, x 16 2.1e8 1470/1490, x 64 8.3e8 2279/2576; 462 (6 + 5) x 1 1.9e8 1581/1465, x 4 7.7e8 1837/2796; 924
+// (6 + 6) x 1 1.1e9 1340/1992. Not measured, and on the pair kernels: spaces of fewer than kStringDetsMin or more
+// than kStringDetsMax determinants.
+constexpr double kStringWork = 3.0e8;
+constexpr int kStringDetsMin = 100, kStringDetsMax = 4096;
 constexpr int kStringRowsZ = 8;         // rows of f and sigma per workgroup of the response sum
 constexpr int kStringPairSegment = 128; // determinants per wavefront of k_string_pairs (512 in large spaces)
 // Pairs left to the list kernels, energy and gradient: those whose regular inverse form loses digits, so that
