@@ -391,6 +391,7 @@ def main():
     batch_grad0 = gb_dev[: cfg["n_act"] * cfg["n_bf"]].cpu().numpy().reshape(cfg["n_act"], cfg["n_bf"])
     batch_consistency = dict(abs_dE_slot0_vs_plain=abs(float(energies[0]) - energy),
                              grad_max_diff_slot0_vs_plain=float(np.abs(batch_grad0 - grad).max()))
+    string_slots, listed_pairs = pool.string_form()
     pool.close()
 
     # ---- rooflines of the single kernels timed on the engine stream (K problems per launch) ----
@@ -417,12 +418,13 @@ def main():
         "k_gep_wave": (mean["eigensolve_ms"], "mfma", K * 10.0 * topo.n_structures ** 3, "TFLOP/s",
                        "latency: per-step LDS round trips, wave reductions and serial recurrences"),
     }
-    # the determinant strings replace the pair kernels where every slot allows it (nothing then runs between the
-    # events around the pair kernels' adjoint): several kernels each way, reported as phases without a roofline
-    strings = mean["pair_backward_adjoint_ms"] < 0.05 * mean["pair_backward_field_ms"]
+    # the determinant strings replace the lane kernels slot by slot: several kernels each way, reported as phases
+    # without a roofline
+    strings = string_slots > 0
     if strings:
         kernels = {k: v for k, v in kernels.items() if not k.startswith("k_pairs_lane")}
-    determinant_form = dict(form="strings" if strings else "pairs", forward_ms=mean["pair_forward_ms"],
+    determinant_form = dict(form="strings" if strings else "pairs", string_slots=string_slots,
+                            listed_pairs=listed_pairs, forward_ms=mean["pair_forward_ms"],
                             backward_ms=mean["pair_backward_ms"],
                             pairwise_flops_per_direction=f_det)
     traffic_table = {}

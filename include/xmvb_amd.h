@@ -298,6 +298,11 @@ int vbe_pool_state_energies(vbe_pool* pool, int32_t slot, double* E_states);
 /* Count of determinant pairs whose overlap block was rank deficient in the last evaluation. */
 int vbe_last_singular_pairs(const vbe_problem* prob, int64_t* count);
 
+/* How the last finished launch evaluated the determinant pairs: the number of its slots (problems) that took the
+ * string form, and the pairs of those slots left to the pair kernels. */
+int vbe_last_string_form(const vbe_problem* prob, int64_t* slots, int64_t* listed);
+int vbe_pool_string_form(const vbe_pool* pool, int64_t* slots, int64_t* listed);
+
 /* ---- batched and served evaluation: pools of resident problems ------------------------------
  * No reference counterpart: the reference evaluates one problem per process. A pool holds
  * `capacity` resident problem slots sharing one structure topology (same active space and

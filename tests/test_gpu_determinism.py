@@ -23,7 +23,8 @@ def _same(a, b):
     ("COV", 10, 120, 360, 0, None),   # medium: lane kernels, private wavefront accumulators
     ("COV", 10, 60, 120, 1, 1.0e3),   # many pairs deferred to the lane-group kernel
     ("COV", 6, 30, 90, 2, 0.0),       # every pair on the lane-group kernel
-    ("COV", 12, 48, 96, 3, None),     # 6x6 blocks: shared W taken in turns, tiles flushed in turns
+    ("COV", 12, 48, 96, 3, None),     # string form, listed pairs on the lane-group kernel
+    ("COV", 12, 48, 96, 3, 9.9e4),    # 6x6 blocks: shared W taken in turns, tiles flushed in turns
     ("FULL", 6, 24, 60, 4, None),
 ])
 def test_repeated_evaluations_are_bitwise_equal(kw, n_act, n_bf, n_aux, seed, limit):
@@ -59,10 +60,13 @@ def test_singular_pairs_are_bitwise_reproducible():
     ctx.close()
 
 
-def test_batched_launch_is_bitwise_reproducible():
+@pytest.mark.parametrize("limit", [None, 9.9e4])  # string form, pair kernels
+def test_batched_launch_is_bitwise_reproducible(limit):
     topo = vb.Topology.build("COV", 10, 10, 1)
     K = 8
     ctx = vb.Context(0)
+    if limit is not None:
+        ctx.set_pair_condition_limit(limit)
     pool = vb.Pool(ctx, topo, capacity=K)
     sps = [vb.synthetic_problem(50 + s, 120, 10, 360) for s in range(K)]
     for s, sp in enumerate(sps):
@@ -70,6 +74,7 @@ def test_batched_launch_is_bitwise_reproducible():
     print("case repeat batched medium x8", flush=True)
     e0, g0 = pool.evaluate(list(range(K)), [sp.C for sp in sps])
     e1, g1 = pool.evaluate(list(range(K)), [sp.C for sp in sps])
+    assert pool.string_form()[0] == (K if limit is None else 0)
     assert _same(e0, e1)
     for a, b in zip(g0, g1):
         assert _same(a, b)
@@ -103,17 +108,23 @@ def test_optimizer_iterates_alone_equal_batched(n_act, n_bf, n_aux, iterations):
     ctx.close()
 
 
-def test_seven_electron_blocks_reproduce_to_rounding():
-    """n_act = 14 with 7-electron blocks: the packed-kernel adjoint has no room in LDS for per-
-    wavefront copies, so it keeps shared atomics; the energy is still the same bits (the forward
-    has no accumulation) and the gradient agrees to rounding."""
-    print("case repeat 7x7 blocks n_act=14", flush=True)
+@pytest.mark.parametrize("limit", [None, 9.9e4])  # string form, pair kernels
+def test_seven_electron_blocks_reproduce_to_rounding(limit):
+    """n_act = 14 with 7-electron blocks: the packed-kernel adjoint of the pair kernels has no room in LDS
+    for per-wavefront copies, so it keeps shared atomics; the energy is still the same bits (the forward
+    has no accumulation) and the gradient agrees to rounding. The string form sums in a fixed order."""
+    print(f"case repeat 7x7 blocks n_act=14 limit={limit}", flush=True)
     sp = vb.synthetic_problem(5, 28, 14, 56)
     topo = vb.Topology.build("COV", 14, 14, 1)
     ctx = vb.Context(0)
+    if limit is not None:
+        ctx.set_pair_condition_limit(limit)
     prob = vb.Problem.from_synthetic(ctx, sp, topo)
     runs = [prob.evaluate(sp.C) for _ in range(2)]
+    assert prob.string_form()[0] == (1 if limit is None else 0)
     assert runs[1][0] == runs[0][0]
+    if limit is None:
+        assert _same(runs[1][1], runs[0][1])
     assert float(np.abs(runs[1][1] - runs[0][1]).max()) <= 1e-12 * max(1.0, float(np.abs(runs[0][1]).max()))
     prob.close()
     ctx.close()

@@ -30,22 +30,30 @@ def case():
     return gold, sp, topo
 
 
-@pytest.fixture(scope="module")
-def fp64_result(case):
-    gold, sp, topo = case
-    print("case precision n_act=14 n_bf=400 n_aux=1200 seed=0 fp64", flush=True)
+def evaluate_fp64(sp, topo, limit=None):
+    print(f"case precision n_act=14 n_bf=400 n_aux=1200 seed=0 fp64 limit={limit}", flush=True)
     ctx = vb.Context(0)
+    if limit is not None:
+        ctx.set_pair_condition_limit(limit)
     prob = vb.Problem.from_synthetic(ctx, sp, topo)
     e, g = prob.evaluate(sp.C)
     mid = prob.intermediates()
+    assert prob.string_form()[0] == (1 if limit is None else 0)
     prob.close()
     ctx.close()
     return e, g, mid
 
 
-def test_precision_fp64_matches_oracle(case, fp64_result):
+@pytest.fixture(scope="module")
+def fp64_result(case):
     gold, sp, topo = case
-    e, g, mid = fp64_result
+    return evaluate_fp64(sp, topo)
+
+
+@pytest.mark.parametrize("limit", [None, 9.9e4])  # string form, pair kernels
+def test_precision_fp64_matches_oracle(case, fp64_result, limit):
+    gold, sp, topo = case
+    e, g, mid = fp64_result if limit is None else evaluate_fp64(sp, topo, limit)
     print(f"dE={abs(e - float(gold['energy'])):.2e} dg={np.abs(g - gold['grad']).max():.2e}", flush=True)
     assert abs(e - float(gold["energy"])) <= E_TOL
     assert np.abs(g - gold["grad"]).max() <= G_TOL

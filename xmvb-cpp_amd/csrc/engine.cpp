@@ -230,6 +230,7 @@ struct vbe_pool {
     int next_ticket = 0;
     int last_lane = 0;
     int64_t last_singular = 0;
+    int64_t last_string_slots = 0, last_listed = 0;  // slots in the string form and their listed pairs
     vbe_phase_times times{};
     // pair-kernel blocks per launch (all listed slots together), chosen by vbe_pool_autotune:
     // forward one-pair-per-lane blocks (the lane-group kernel takes twice this), backward blocks
@@ -861,6 +862,11 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
     return ms;
 }
 
+// string_slot (device.hpp) of a launch's flags
+bool in_string_form(const int* f) {
+    return f[xmvb_amd::FLAG_STRINGS] && f[xmvb_amd::FLAG_NEAR] <= xmvb_amd::kStringListMax;
+}
+
 // Wait for a lane, record phase times, raise on device flags (or, with slot_status, report each
 // listed slot's status instead of raising).
 void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
@@ -883,13 +889,17 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
         t.pair_backward_field_ms = lane.with_grad ? elapsed(lane.ev[EV_BWD_BEGIN], lane.ev[EV_BWD_FIELD]) : 0.f;
         t.pair_backward_adjoint_ms = lane.with_grad ? elapsed(lane.ev[EV_BWD_FIELD], lane.ev[EV_BWD_ADJOINT]) : 0.f;
     }
-    int64_t singular = 0;
+    int64_t singular = 0, string_slots = 0, listed = 0;
     std::string err;
     int status = VBE_OK;
     if (slot_status) slot_status->assign(lane.slots.size(), VBE_OK);
     for (size_t i = 0; i < lane.slots.size(); ++i) {
         const int* f = lane.h_flags + FLAG_COUNT * i;
         singular += f[FLAG_SINGULAR_PAIRS];
+        if (in_string_form(f)) {
+            ++string_slots;
+            listed += f[FLAG_DEFERRED];
+        }
         const int si = f[FLAG_NORMALIZATION] || f[FLAG_ACTIVE_OVERLAP] || f[xmvb_amd::FLAG_EIGEN] ? VBE_ERR_NUMERIC
                        : f[FLAG_METRIC]                                                        ? VBE_ERR_METRIC
                                                                                                : VBE_OK;
@@ -913,6 +923,8 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
             err = "structure metric is not positive definite" + where;
     }
     p->last_singular = singular;
+    p->last_string_slots = string_slots;
+    p->last_listed = listed;
     if (status != VBE_OK && !slot_status) throw StatusError(status, err);
 }
 
@@ -937,10 +949,9 @@ void evaluate_now(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, boo
     check(hipEventSynchronize(lane.done), "hipEventSynchronize");
     bool pairs = false, strings = false;
     for (size_t i = 0; i < in.size(); ++i) {
-        const int* f = lane.h_flags + FLAG_COUNT * i;
-        const bool string_slot = f[xmvb_amd::FLAG_STRINGS] && f[xmvb_amd::FLAG_NEAR] <= xmvb_amd::kStringListMax;
-        strings = strings || string_slot;
-        pairs = pairs || !string_slot;
+        const bool s = in_string_form(lane.h_flags + FLAG_COUNT * i);
+        strings = strings || s;
+        pairs = pairs || !s;
     }
     p->pair_hold = pairs ? kPairHold : std::max(p->pair_hold - 1, 0);
     const bool missing = (strings && !lane.string_kernels) || (pairs && !lane.pair_kernels);
@@ -1810,6 +1821,17 @@ int vbe_last_phase_times(const vbe_problem* prob, vbe_phase_times* times) {
     if (!prob || !times) return VBE_ERR_ARGUMENT;
     *times = prob->pool->times;
     return VBE_OK;
+}
+
+int vbe_pool_string_form(const vbe_pool* pool, int64_t* slots, int64_t* listed) {
+    if (!pool || !slots || !listed) return VBE_ERR_ARGUMENT;
+    *slots = pool->last_string_slots;
+    *listed = pool->last_listed;
+    return VBE_OK;
+}
+
+int vbe_last_string_form(const vbe_problem* prob, int64_t* slots, int64_t* listed) {
+    return prob ? vbe_pool_string_form(prob->pool.get(), slots, listed) : VBE_ERR_ARGUMENT;
 }
 
 int vbe_last_singular_pairs(const vbe_problem* prob, int64_t* count) {

@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "vbe_context_create", "vbe_context_destroy", "vbe_last_error", "vbe_global_error", "vbe_problem_upload",
     "vbe_problem_release", "vbe_problem_device_bytes", "vbe_eval", "vbe_eval_device", "vbe_eval_forward",
     "vbe_complete_gradient", "vbe_last_intermediates", "vbe_last_phase_times", "vbe_last_singular_pairs",
+    "vbe_last_string_form", "vbe_pool_string_form",
     "vbe_pool_create", "vbe_pool_destroy", "vbe_pool_load", "vbe_pool_device_bytes", "vbe_pool_unload",
     "vbe_context_memory", "vbe_pool_autotune", "vbe_pool_eval_device",
     "vbe_pool_submit", "vbe_pool_wait", "vbe_pool_poll", "vbe_pool_phase_times", "vbe_set_pair_condition_limit", "vbe_set_ri_precision",
@@ -156,6 +157,8 @@ def library() -> C.CDLL:
         lib.vbe_last_intermediates.argtypes = [P, P, P, P, P, P, P, P]
         lib.vbe_last_phase_times.argtypes = [P, C.POINTER(PhaseTimes)]
         lib.vbe_last_singular_pairs.argtypes = [P, C.POINTER(I64)]
+        lib.vbe_last_string_form.argtypes = [P, C.POINTER(I64), C.POINTER(I64)]
+        lib.vbe_pool_string_form.argtypes = [P, C.POINTER(I64), C.POINTER(I64)]
         lib.vbe_pool_create.argtypes = [P, C.POINTER(TopologyView), I32, I32, I32, I32, C.POINTER(P)]
         lib.vbe_pool_destroy.argtypes = [P]
         lib.vbe_pool_destroy.restype = None
@@ -550,6 +553,12 @@ class Problem:
         self.ctx._lib.vbe_last_phase_times(self._h, C.byref(t))
         return {name: getattr(t, name) for name, _ in PhaseTimes._fields_}
 
+    def string_form(self) -> tuple:
+        """(1 if the last launch took the string form else 0, its pairs left to the pair kernels)."""
+        s, n = C.c_int64(), C.c_int64()
+        self.ctx._lib.vbe_last_string_form(self._h, C.byref(s), C.byref(n))
+        return s.value, n.value
+
     def singular_pairs(self) -> int:
         c = C.c_int64()
         self.ctx._lib.vbe_last_singular_pairs(self._h, C.byref(c))
@@ -681,6 +690,12 @@ class Pool:
         out = np.zeros(self.n_states)
         self.ctx.check(self.ctx._lib.vbe_pool_state_energies(self._h, slot, _ptr(out)))
         return out
+
+    def string_form(self) -> tuple:
+        """(slots of the last finished launch in the string form, their pairs left to the pair kernels)."""
+        s, n = C.c_int64(), C.c_int64()
+        self.ctx._lib.vbe_pool_string_form(self._h, C.byref(s), C.byref(n))
+        return s.value, n.value
 
     def phase_times(self) -> dict:
         t = PhaseTimes()
