@@ -553,7 +553,10 @@ __global__ void __launch_bounds__(256) k_string_pairs(const SlotDesc* __restrict
         h += __shfl_xor(h, 16, 64);
         h += __shfl_xor(h, 32, 64);
         h += ka * mb + ma * kb;
-        if (d.det >= 0 && order_couple(base + i16, topo.flip != nullptr) <= couple && (k4 < 2 || topo.flip)) {
+        // Where e is its own partner, d and its partner (i16 and i16 + 8) have the same four elements, equal but for
+        // rounding: the first writes them, else the order of the lanes' stores would choose.
+        const bool writes = fe != e || d.flip == d.det || i16 < 8;
+        if (d.det >= 0 && writes && order_couple(base + i16, topo.flip != nullptr) <= couple && (k4 < 2 || topo.flip)) {
             const int p = k4 < 2 ? d.det : d.flip, q = k4 < 2 ? e : fe;
             const size_t at = k4 & 1 ? (size_t)q + (size_t)n_det * p : (size_t)p + (size_t)n_det * q;
             Hd[at] = h;
