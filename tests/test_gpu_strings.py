@@ -321,3 +321,40 @@ def test_selected_states(kw, n_act, mult, states):
     ref = oracle.evaluate(26, 40, topo, sp.S, sp.h, sp.B, sp.C, states=idx, weights=w)
     assert abs(e - e2) <= E_TOL and abs(e - ref["energy"]) <= 1e-8
     assert np.abs(g - g2).max() <= G_TOL and np.abs(g - ref["grad"]).max() <= 1e-7
+
+
+def test_string_arrays_give_way_to_slots():
+    """Two slots of 12 orbitals (30 MB of string arrays each) under budgets that leave out the arrays of one and of both:
+    the slots load as they would without the string form, and the pair kernels serve what has none."""
+    topo = vb.Topology.build("COV", 12, 12, 1)
+    sps = [vb.synthetic_problem(70 + k, 30, 12, 45) for k in range(2)]
+
+    def run(budget):
+        ctx = vb.Context(0, budget)
+        pool = vb.Pool(ctx, topo, 2)
+        for k, sp in enumerate(sps):
+            pool.load_synthetic(k, sp)
+        used = ctx.memory()[0]
+        assert used == pool.device_bytes()
+        forms, values = [], []
+        for k, sp in enumerate(sps):
+            e, g = pool.evaluate([k], [sp.C])
+            values.append((e[0], g[0]))
+            forms.append(pool.string_form()[0])
+        pool.close()
+        ctx.close()
+        return used, forms, values
+
+    full, forms, ref = run(0)
+    assert forms == [1, 1]
+    slack = 4 << 20  # staging of the evaluations
+    one, forms, values = run(full - 1)
+    arrays = full - one
+    assert arrays > 4 * slack and forms == [1, 0]
+    for budget, want in ((full - arrays + slack, [1, 0]), (full - 2 * arrays + slack, [0, 0])):
+        used, forms, got = run(budget)
+        assert used <= budget and forms == want
+        values += got
+    for at, (e, g) in enumerate(values):
+        assert abs(e - ref[at % 2][0]) <= 1e-9
+        assert np.linalg.norm(g - ref[at % 2][1]) <= 1e-9 * np.linalg.norm(ref[at % 2][1])

@@ -79,6 +79,7 @@ struct vbe_context {
     // synchronizing a shared stream.
     std::vector<hipStream_t> streams;
     int next_stream = 0;
+    std::vector<vbe_pool*> pools;  // every pool, for release_string_memory
     hipStream_t take_stream() {
         std::lock_guard<std::mutex> g(mu);
         if (streams.empty()) {
@@ -107,27 +108,38 @@ struct vbe_context {
 
 namespace {
 
-// Device allocations charged to a context budget.
+// Gives back the separate string-form arrays of the context's pools (defined below). false: none were held.
+bool release_string_memory(vbe_context* ctx);
+
+// Device allocations charged to a context budget. One that does not fit takes the string form's arrays back first;
+// an optional one (those arrays themselves) does not.
 struct DeviceArena {
     vbe_context* ctx = nullptr;
     std::vector<void*> ptrs;
     uint64_t bytes = 0;
     template <typename T>
-    T* alloc(size_t count) {
+    T* alloc(size_t count, bool optional = false) {
         const size_t nbytes = std::max<size_t>(count, 1) * sizeof(T);
-        {
-            std::lock_guard<std::mutex> g(ctx->mu);
-            if (ctx->budget && ctx->in_use + nbytes > ctx->budget)
-                throw StatusError(VBE_ERR_MEMORY, "HBM budget exceeded while allocating problem storage");
-            ctx->in_use += nbytes;  // reserved before the allocation, returned if it fails
-        }
         void* p = nullptr;
-        const hipError_t e = hipMalloc(&p, nbytes);
-        if (e != hipSuccess) {
-            std::lock_guard<std::mutex> g(ctx->mu);
-            ctx->in_use -= std::min(ctx->in_use, (uint64_t)nbytes);
+        hipError_t e = hipErrorOutOfMemory;
+        for (bool last = optional;; last = true) {
+            bool fits;
+            {
+                std::lock_guard<std::mutex> g(ctx->mu);
+                fits = !ctx->budget || ctx->in_use + nbytes <= ctx->budget;
+                if (fits) ctx->in_use += nbytes;  // reserved before the allocation, returned if it fails
+            }
+            if (fits) {
+                e = hipMalloc(&p, nbytes);
+                if (e == hipSuccess) break;
+                (void)hipGetLastError();  // not for the next call to find
+                std::lock_guard<std::mutex> g(ctx->mu);
+                ctx->in_use -= std::min(ctx->in_use, (uint64_t)nbytes);
+            }
+            if (!last && release_string_memory(ctx)) continue;
+            if (!fits) throw StatusError(VBE_ERR_MEMORY, "HBM budget exceeded while allocating problem storage");
+            check(e, "hipMalloc");
         }
-        check(e, "hipMalloc");
         ptrs.push_back(p);
         bytes += nbytes;
         return static_cast<T*>(p);
@@ -149,6 +161,7 @@ struct Slot {
     int n_bf = 0, n_aux = 0;
     double e_nuc = 0.0;
     std::unique_ptr<DeviceArena> arena;
+    std::unique_ptr<DeviceArena> string_arena;  // arrays of the string form that do not fit the partial rows
     SlotDesc desc{};           // workspace + static pointers; per-launch fields filled at launch
     std::vector<double> S_host;  // AO overlap (the optimiser's chart metric)
     bool has_root = false;     // desc.coef holds this slot's last structure eigenvector
@@ -237,6 +250,7 @@ struct vbe_pool {
     int fwd_target = kLaneBlocks;
     int bwd_target = kLaneBlocks;
     int pair_hold = 1;  // launches left that include the pair kernels from the start (evaluate_now)
+    bool retains = false;  // a forward evaluation may wait for its gradient (a problem's pool)
     int pair_run = 0;   // launches in a row that no slot's string form served; below zero: launches to wait first
 
     // serializes host access to the pool's lanes and slots between the caller's thread and the
@@ -244,6 +258,11 @@ struct vbe_pool {
     std::recursive_mutex mu;
 
     ~vbe_pool() {
+        if (ctx) {
+            std::lock_guard<std::mutex> g(ctx->mu);
+            std::erase(ctx->pools, this);
+        }
+        const std::lock_guard<std::recursive_mutex> lk(mu);  // release_string_memory may still hold it
         for (auto& l : lanes) {
             if (l.done) (void)hipEventSynchronize(l.done);  // the lane's last launch (streams are shared)
             for (auto& e : l.ev)
@@ -342,13 +361,46 @@ int bwd_blocks_cap(const vbe_pool* p) {
     return (int)std::min<long long>(kMaxBwdBlocksPerSlot, std::max<long long>(1, (pair_count(p) + 7) / 8));
 }
 
+// kStringWork's measure of a launch of `count` problems
+double string_work(const vbe_pool* p, long long count) {
+    const double pair = (double)p->topo.n_det * p->n_alpha * p->n_beta;
+    return pair * pair * (double)count;
+}
+
+// Those slots stay on the pair kernels until they are loaded again. A pool in use by another thread, and one whose
+// forward evaluation may still be differentiated (a single problem's), keep theirs.
+bool release_string_memory(vbe_context* ctx) {
+    std::vector<std::unique_lock<std::recursive_mutex>> held;
+    std::vector<vbe_pool*> pools;
+    {
+        std::lock_guard<std::mutex> g(ctx->mu);
+        for (vbe_pool* p : ctx->pools) {
+            std::unique_lock<std::recursive_mutex> lk(p->mu, std::try_to_lock);
+            if (!lk || p->retains) continue;
+            held.push_back(std::move(lk));
+            pools.push_back(p);
+        }
+    }
+    bool any = false;
+    for (vbe_pool* p : pools) {
+        for (auto& l : p->lanes) check(hipEventSynchronize(l.done), "hipEventSynchronize");  // launches that use them
+        for (auto& s : p->slots) {
+            if (!s.string_arena) continue;
+            s.string_arena.reset();
+            s.desc.sw = xmvb_amd::StringWork{};
+            any = true;
+        }
+    }
+    return any;
+}
+
 // Device copies of the string form's tables. The host vectors must outlive the stream's copies.
 void upload_string_tables(const xmvb_amd::StringTables& h, DeviceArena& A, xmvb_amd::StringTopo& d, hipStream_t st) {
     d = xmvb_amd::StringTopo{};
     if (!h.enabled) return;
     auto put = [&](auto& dst, const auto& v) {
         using E = std::remove_cv_t<std::remove_reference_t<decltype(v[0])>>;
-        E* p = A.alloc<E>(v.size());
+        E* p = A.alloc<E>(v.size(), true);
         if (!v.empty()) upload(p, v.data(), v.size(), st);
         dst = p;
     };
@@ -531,13 +583,23 @@ std::unique_ptr<vbe_pool> make_pool(vbe_context* ctx, const vbe_topology_view& t
         if (T.state_idx[k] >= ns)
             throw StatusError(VBE_ERR_ARGUMENT, "selected state " + std::to_string(T.state_idx[k]) +
                                                     " is out of range for " + std::to_string(ns) + " structures");
-    xmvb_amd::StringTables tables =
-        xmvb_amd::build_string_tables(n_act, n_alpha, n_beta, nd, t.alpha_masks, t.det_alpha, t.beta_masks, t.det_beta,
-                                      off.data(), t.term_structure, t.term_coefficient, flip);
-    upload_string_tables(tables, A, T.str, st);
+    // only where some launch of the pool may take the string form (shape_for)
+    xmvb_amd::StringTables tables;
+    if (xmvb_amd::pairs_lane_supported(n_alpha, n_beta, true) && string_work(p.get(), capacity) >= xmvb_amd::kStringWork)
+        tables = xmvb_amd::build_string_tables(n_act, n_alpha, n_beta, nd, t.alpha_masks, t.det_alpha, t.beta_masks,
+                                               t.det_beta, off.data(), t.term_structure, t.term_coefficient, flip);
+    try {
+        upload_string_tables(tables, A, T.str, st);
+    } catch (const StatusError&) {
+        T.str = xmvb_amd::StringTopo{};  // no room: the pair kernels alone
+    }
     check(xmvb_amd::configure_kernels(n_act, T.ng, ns, std::max(n_alpha, n_beta)), "hipFuncSetAttribute");
     check(hipStreamSynchronize(st), "hipStreamSynchronize");
     p->slots.resize(capacity);
+    {
+        std::lock_guard<std::mutex> g(ctx->mu);
+        ctx->pools.push_back(p.get());
+    }
     return p;
 }
 
@@ -556,9 +618,9 @@ void check_slots_free(const vbe_pool* p, const int* slots, int count) {
 // aligned to 256 bytes). With base == nullptr nothing is assigned and only the size is returned.
 // The slot's own arena and the no-allocation entry point's static scratch use this same layout.
 // The string form's arrays lie over the partial rows of the lane kernels where they fit (a slot uses one
-// or the other; the front rows hold the listed pairs'), else behind everything else; strings = false
-// leaves them out.
-size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* base, SlotDesc& d, bool strings = true) {
+// or the other; the front rows hold the listed pairs'), else behind everything else where append is set, or
+// nowhere (sw.Sinv null).
+size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* base, SlotDesc& d, bool append) {
     const TopoDesc& T = p->topo;
     const size_t n = T.n, np = T.np, nd = T.n_det, ns = T.n_str;
     size_t off = 0;
@@ -601,13 +663,14 @@ size_t carve_workspace(const vbe_pool* p, int n_bf, int n_aux, unsigned char* ba
     take(d.chunk_count,
          (size_t)(std::max<long long>(T.n_lane_pairs, pair_count(p)) / xmvb_amd::kCompactChunk + 2));
     if (base) d.sw = xmvb_amd::StringWork{};
-    if (strings && T.str.enabled) {
+    if (T.str.enabled) {
         xmvb_amd::StringWork unused{};
         const size_t count = xmvb_amd::string_work_carve(T, nullptr, unused);
         const size_t front = ((size_t)(xmvb_amd::kListBlocks + xmvb_amd::kSingularBlocks) * len + 31) / 32 * 32;
-        double* work = base ? d.partials + front : nullptr;
-        if (front + count > partial_rows) take(work, count);
-        if (base) (void)xmvb_amd::string_work_carve(T, work, d.sw);
+        double* work = nullptr;
+        if (front + count <= partial_rows) work = base ? d.partials + front : nullptr;
+        else if (append) take(work, count);
+        if (base && work) (void)xmvb_amd::string_work_carve(T, work, d.sw);
     }
     return (off + 255) & ~size_t(255);
 }
@@ -647,6 +710,7 @@ void load_slot(vbe_pool* p, int slot, int n_bf, int n_aux, const double* S, cons
     s.loaded = false;
     if (realloc) {
         s.arena.reset();
+        s.string_arena.reset();
         s.desc = SlotDesc{};
         s.C_buf = s.grad_buf = nullptr;
         s.support_buf = nullptr;
@@ -670,8 +734,8 @@ void load_slot(vbe_pool* p, int slot, int n_bf, int n_aux, const double* S, cons
         d.b_tiled = tiled ? 1 : 0;
         // the per-evaluation workspace as one block, in the layout the no-allocation entry point
         // reproduces in its static scratch
-        unsigned char* ws = A.alloc<unsigned char>(carve_workspace(p, n_bf, n_aux, nullptr, d));
-        carve_workspace(p, n_bf, n_aux, ws, d);
+        unsigned char* ws = A.alloc<unsigned char>(carve_workspace(p, n_bf, n_aux, nullptr, d, false));
+        carve_workspace(p, n_bf, n_aux, ws, d, false);
         double* C_buf = A.alloc<double>(n * n_bf);
         double* grad_buf = A.alloc<double>(n * n_bf);
         uint8_t* support_buf = A.alloc<uint8_t>(n * n_bf);
@@ -680,6 +744,18 @@ void load_slot(vbe_pool* p, int slot, int n_bf, int n_aux, const double* S, cons
         s.grad_buf = grad_buf;
         s.support_buf = support_buf;
         s.desc = d;
+    }
+    if (p->topo.str.enabled && !s.desc.sw.Sinv) {
+        // the pair kernels serve the slot where these arrays do not fit
+        auto arena = std::make_unique<DeviceArena>();
+        arena->ctx = p->ctx;
+        xmvb_amd::StringWork sw{};
+        try {
+            double* work = arena->alloc<double>(xmvb_amd::string_work_carve(p->topo, nullptr, sw), true);
+            (void)xmvb_amd::string_work_carve(p->topo, work, s.desc.sw);
+            s.string_arena = std::move(arena);
+        } catch (const StatusError&) {
+        }
     }
     s.n_bf = n_bf;
     s.n_aux = n_aux;
@@ -710,12 +786,6 @@ void load_slot(vbe_pool* p, int slot, int n_bf, int n_aux, const double* S, cons
     }
     check(hipStreamSynchronize(st), "hipStreamSynchronize");
     s.loaded = true;
-}
-
-// kStringWork's measure of a launch of `count` problems
-double string_work(const vbe_pool* p, long long count) {
-    const double pair = (double)p->topo.n_det * p->n_alpha * p->n_beta;
-    return pair * pair * (double)count;
 }
 
 // Per-slot inputs of one launch.
@@ -1113,7 +1183,7 @@ int eval_device_in_scratch(vbe_context* ctx, vbe_problem* prob, const double* d_
         if (!s.loaded) throw StatusError(VBE_ERR_ARGUMENT, "problem not loaded");
         SlotDesc ws = s.desc;
         // without the string form where its arrays do not fit
-        const bool strings = carve_workspace(p, s.n_bf, s.n_aux, nullptr, ws) <= scratch_bytes;
+        const bool strings = carve_workspace(p, s.n_bf, s.n_aux, nullptr, ws, true) <= scratch_bytes;
         const size_t need = carve_workspace(p, s.n_bf, s.n_aux, nullptr, ws, strings);
         if (need > scratch_bytes)
             throw StatusError(VBE_ERR_MEMORY, "evaluation workspace of " + std::to_string(need) +
@@ -1402,6 +1472,7 @@ int vbe_pool_unload(vbe_pool* pool, int32_t slot) {
         // (no pending submission holds it); a synchronous evaluation returns only when done
         Slot& s = pool->slots[slot];
         s.arena.reset();
+        s.string_arena.reset();
         s.desc = SlotDesc{};
         s.C_buf = s.grad_buf = nullptr;
         s.support_buf = nullptr;
@@ -1426,7 +1497,8 @@ int vbe_pool_device_bytes(const vbe_pool* pool, uint64_t* bytes) {
     if (!pool || !bytes) return VBE_ERR_ARGUMENT;
     uint64_t b = pool->topo_arena.bytes + pool->ri_stage_arena.bytes + pool->opt_arena.bytes;
     for (const auto& s : pool->slots)
-        if (s.arena) b += s.arena->bytes;
+        for (const auto* a : {s.arena.get(), s.string_arena.get()})
+            if (a) b += a->bytes;
     *bytes = b;
     return VBE_OK;
 }
@@ -1617,6 +1689,7 @@ int vbe_problem_upload(vbe_context* ctx, const vbe_dims* dims, const double* S_a
         if (dims->n_bf <= 0 || dims->n_aux <= 0) throw StatusError(VBE_ERR_ARGUMENT, "dimensions must be positive");
         auto prob = std::make_unique<vbe_problem>();
         prob->pool = make_pool(ctx, *topo, dims->n_act, dims->n_alpha, dims->n_beta, 1);
+        prob->pool->retains = true;
         load_slot(prob->pool.get(), 0, dims->n_bf, dims->n_aux, S_ao, h_ao, B_packed, e_nuc);
         check(hipHostMalloc(reinterpret_cast<void**>(&prob->stage), 2 * sizeof(double) * dims->n_act * dims->n_bf,
                             hipHostMallocDefault),

@@ -53,7 +53,7 @@ StringTables build_string_tables(int n, int n_alpha, int n_beta, int n_det, cons
                                  const double* tc, const std::vector<int>& flip) {
     StringTables t;
     t.n = n;
-    if (n > 14 || n_alpha < 1 || n_beta < 1 || n_alpha > 8 || n_beta > 8 || n_alpha >= n ||
+    if (n > 14 || n_alpha < 1 || n_beta < 1 || n_alpha > 7 || n_beta > 7 || n_alpha >= n ||
         n_beta >= n || n_det < kStringDetsMin || n_det > kStringDetsMax)
         return t;
     t.rank.assign(1u << n, 0);

@@ -1250,7 +1250,7 @@ int z_blocks(const StringTopo& t) { return (t.a.N + kStringRowsZ - 1) / kStringR
 
 template <int M>
 void minors(hipStream_t st, const SlotDesc* slots, unsigned z, int n, const StringSpace& sp, bool beta) {
-    if constexpr (M > 8) return;
+    if constexpr (M > 7) return;  // the lane kernels' shapes
     else if (sp.m == M) {
         hipLaunchKernelGGL(k_string_minors<M>, dim3(blocks_for(sp.N), (unsigned)((sp.N + kMinorRows - 1) / kMinorRows), z),
                            dim3(256), 0, st, slots, n, sp, beta);
