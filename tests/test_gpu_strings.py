@@ -134,15 +134,15 @@ def test_ill_conditioned_orbitals_keep_the_pair_kernels_in_a_mixed_launch():
 
 
 class Waited:
-    """One 12-orbital problem through every call that waits for its launch: those choose which kernels to enqueue from
-    the launches before and repeat a launch whose slots needed the others."""
+    """One 12-orbital problem through every way to evaluate it: each launch takes the kernels that the launches before
+    needed and is repeated where its slots needed the others."""
 
     def __init__(self, call):
         self.topo = vb.Topology.build("COV", 12, 12, 1)
         self.sp = vb.synthetic_problem(77, 30, 12, 45)
         self.call = call
         self.ctx = vb.Context(0)
-        if call == "pool":
+        if call in ("pool", "submit", "scheduler"):
             self.pool = vb.Pool(self.ctx, self.topo, 1)
             self.pool.load_synthetic(0, self.sp)
         else:
@@ -154,6 +154,22 @@ class Waited:
         if self.call == "two_phase":
             e = self.prob.evaluate_forward(C)
             return e, self.prob.complete_gradient(), self.prob.string_form()[0]
+        if self.call == "submit":  # the repetition happens at the poll or at the wait
+            ticket = self.pool.submit([0], [C])
+            self.polled = not getattr(self, "polled", False)
+            while self.polled and not self.pool.poll(ticket):
+                pass
+            e, g = self.pool.wait(ticket)
+            return e[0], g[0], self.pool.string_form()[0]
+        if self.call == "scheduler":
+            g = np.full(C.shape, np.nan)
+            sched = vb.Scheduler(self.ctx)
+            sched.submit(self.pool, 0, C, g)
+            done = []
+            while not done:
+                done = sched.collect(wait_us=100000)
+            sched.close()
+            return done[0]["energy"], g, self.pool.string_form()[0]
         c = torch.from_numpy(np.ascontiguousarray(C)).to("cuda:0")
         g = torch.full_like(c, float("nan"))
         torch.cuda.synchronize()
@@ -166,13 +182,13 @@ class Waited:
         return e, g.cpu().numpy().reshape(C.shape), form
 
     def close(self):
-        (self.pool if self.call == "pool" else self.prob).close()
+        (self.pool if hasattr(self, "pool") else self.prob).close()
         self.ctx.close()
 
 
-@pytest.mark.parametrize("call", ["evaluate", "two_phase", "device", "pool"])
+@pytest.mark.parametrize("call", ["evaluate", "two_phase", "device", "pool", "submit", "scheduler"])
 @pytest.mark.parametrize("order", ["ggi", "ggrg", "gggnig", "iiiiiiggi", "rrrrrgg"])
-def test_waited_launches_repeat_with_the_kernels_they_lack(call, order):
+def test_launches_repeat_with_the_kernels_they_lack(call, order):
     """g: well separated orbitals (string form, after two of them alone); i: ill-conditioned S_act; r: too many rank
     deficient blocks; n: a nearly singular block (listed pairs). Five
     launches without a string slot leave the string kernels out until one has one."""

@@ -170,6 +170,14 @@ struct Slot {
     uint8_t* support_buf = nullptr;
 };
 
+// Per-slot inputs of one launch.
+struct SlotInput {
+    int slot;
+    const double* C;         // device orbitals
+    const uint8_t* support;  // device support mask or null
+    double* grad;            // device gradient output
+};
+
 // Energies (two) and flags of one slot of a launch.
 constexpr size_t kSlotOutBytes = 2 * sizeof(double) + FLAG_COUNT * sizeof(int);
 
@@ -187,7 +195,7 @@ struct Lane {
     int* d_flags = nullptr;
     double* h_energy = nullptr;  // pinned
     int* h_flags = nullptr;      // pinned
-    // a gradient that a single problem's launch also brings back, before its completion point
+    // gradients that the launch also brings back, before its completion point
     const double* back_src = nullptr;
     double* back_dst = nullptr;  // pinned
     size_t back_doubles = 0;
@@ -204,7 +212,12 @@ struct Lane {
     bool events_valid = false;
     bool strings = false;       // the last forward offered the string form
     bool string_kernels = false;  // and launched its kernels
-    bool pair_kernels = true;     // and the pair kernels
+    bool pair_kernels = true;     // and the lane kernels
+    // such a forward until settle() has seen which kernels its slots needed, and what a repetition takes
+    bool unsettled = false;
+    std::vector<SlotInput> inputs;
+    const SlotDesc* ws = nullptr;
+    bool pinned = false, timed = true;
     bool scratch = false;  // the launch ran on a workspace outside the slots (no-allocation entry point)
     int ticket = -1;
     std::vector<int> slots;
@@ -249,7 +262,7 @@ struct vbe_pool {
     // forward one-pair-per-lane blocks (the lane-group kernel takes twice this), backward blocks
     int fwd_target = kLaneBlocks;
     int bwd_target = kLaneBlocks;
-    int pair_hold = 1;  // launches left that include the pair kernels from the start (evaluate_now)
+    int pair_hold = 1;  // launches left that include the lane kernels from the start (launch)
     bool retains = false;  // a forward evaluation may wait for its gradient (a problem's pool)
     int pair_run = 0;   // launches in a row that no slot's string form served; below zero: launches to wait first
 
@@ -788,14 +801,6 @@ void load_slot(vbe_pool* p, int slot, int n_bf, int n_aux, const double* S, cons
     s.loaded = true;
 }
 
-// Per-slot inputs of one launch.
-struct SlotInput {
-    int slot;
-    const double* C;         // device orbitals
-    const uint8_t* support;  // device support mask or null
-    double* grad;            // device gradient output
-};
-
 LaunchShape shape_for(const vbe_pool* p, const std::vector<SlotInput>& in, bool pinned) {
     LaunchShape sh{};
     sh.pinned = pinned;
@@ -856,10 +861,11 @@ LaunchShape shape_for(const vbe_pool* p, const std::vector<SlotInput>& in, bool 
 }
 
 enum class Forms { both, strings, pairs };
+constexpr int kPairHold = 64, kPairRun = 4;
 
 // Enqueue forward and/or backward for a set of slots on a lane, then the D2H of energies and flags.
 // ws (optional, single-slot launches): a descriptor whose workspace replaces the slot's own.
-// forms: where the string form is offered, the kernels of both forms, or of one of them (see evaluate_now).
+// forms: where the string form is offered, the kernels of both forms, or of one of them (see launch).
 // timed: record the phase events (read by finish into the pool's phase times); the optimiser's
 // inner evaluations skip them, a dozen event records per launch being host time on its critical path.
 void enqueue(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
@@ -937,11 +943,67 @@ bool in_string_form(const int* f) {
     return f[xmvb_amd::FLAG_STRINGS] && f[xmvb_amd::FLAG_NEAR] <= xmvb_amd::kStringListMax;
 }
 
+// Enqueue a launch with the kernels that the pool's recent launches needed. Once one has shown that no slot needs
+// the lane kernels (S_act too ill-conditioned, or too many listed pairs), they stay out: their idle launches are
+// 50-60 us of a call. Should a slot then need them, the launch is repeated with them (settle), and the pool
+// takes both until kPairHold launches in a row have needed none. Where kPairRun launches in a row had no slot for
+// the string form at all, its kernels stay out in turn (44 us of 815 for eight ill-conditioned problems of 252
+// determinants), but for the test of S_act: a slot that passes it has the launch repeated. The form of a slot
+// follows from its own S_act in every case.
+void launch(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
+            const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true) {
+    // a repeated Davidson solve would start from what the first one left
+    const bool davidson = p->eigensolver == VBE_EIGENSOLVER_DAVIDSON;
+    const Forms forms = !forward || davidson     ? Forms::both
+                        : p->pair_run >= kPairRun ? Forms::pairs
+                        : p->pair_hold == 0       ? Forms::strings
+                                                  : Forms::both;
+    lane.unsettled = false;
+    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed, forms);
+    if (!forward || !lane.strings) return;
+    lane.unsettled = true;
+    lane.inputs = in;
+    lane.ws = ws;
+    lane.pinned = pinned;
+    lane.timed = timed;
+}
+
+// After a launch has completed: learn from its slots. false: some needed kernels that it left out, and the launch
+// has been enqueued again with all of them.
+bool settle(vbe_pool* p, Lane& lane) {
+    if (!lane.unsettled) return true;
+    bool pairs = false, strings = false;
+    for (size_t i = 0; i < lane.slots.size(); ++i) {
+        const bool s = in_string_form(lane.h_flags + FLAG_COUNT * i);
+        strings = strings || s;
+        pairs = pairs || !s;
+    }
+    p->pair_hold = pairs ? kPairHold : std::max(p->pair_hold - 1, 0);
+    p->pair_run = !strings                ? p->pair_run + (p->pair_run < kPairRun)
+                  : !lane.string_kernels ? -kPairHold
+                                         : std::min(p->pair_run, 0);
+    const bool complete = (!strings || lane.string_kernels) && (!pairs || lane.pair_kernels);
+    if (!complete) {
+        check(hipSetDevice(p->ctx->device), "hipSetDevice");
+        const std::vector<SlotInput> in = lane.inputs;
+        enqueue(p, lane, in, lane.with_grad, true, lane.ws, lane.pinned, lane.timed);
+    }
+    lane.unsettled = false;  // not where the repetition failed: the results are not complete then
+    return complete;
+}
+
 // Wait for a lane, record phase times, raise on device flags (or, with slot_status, report each
 // listed slot's status instead of raising).
 void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
     check(hipEventSynchronize(lane.done), "hipEventSynchronize");
+    try {
+        if (!settle(p, lane)) check(hipEventSynchronize(lane.done), "hipEventSynchronize");
+    } catch (...) {
+        lane.busy = false;
+        throw;
+    }
     lane.busy = false;
+    lane.back_doubles = 0;
     using namespace xmvb_amd;
     if (lane.events_valid) {
         auto& t = p->times;
@@ -998,37 +1060,13 @@ void finish(vbe_pool* p, Lane& lane, std::vector<int>* slot_status = nullptr) {
     if (status != VBE_OK && !slot_status) throw StatusError(status, err);
 }
 
-// A launch that the caller waits for at once: the string form and the list kernels alone, without the idle launches
-// of the lane kernels, once a launch of the pool has shown that no slot needs them (S_act too ill-conditioned,
-// or too many listed pairs). Should a
-// slot then turn out to need them, the launch is repeated with them, and the pool takes both until
-// kPairHold launches in a row have needed none. Where kPairRun launches in a row had no slot for the
-// string form at all, its kernels stay out in turn, but for the test of S_act: a slot that passes it has the launch
-// repeated. The form of a slot follows from its own S_act in every case.
-constexpr int kPairHold = 64, kPairRun = 4;
+// A launch that the caller waits for at once; finish() then has its results.
 void evaluate_now(vbe_pool* p, Lane& lane, const std::vector<SlotInput>& in, bool with_grad, bool forward,
                   const SlotDesc* ws = nullptr, bool pinned = false, bool timed = true) {
-    // a repeated Davidson solve would start from what the first one left
-    const bool davidson = p->eigensolver == VBE_EIGENSOLVER_DAVIDSON;
-    const Forms forms = !forward || davidson     ? Forms::both
-                        : p->pair_run >= kPairRun ? Forms::pairs
-                        : p->pair_hold == 0       ? Forms::strings
-                                                  : Forms::both;
-    enqueue(p, lane, in, with_grad, forward, ws, pinned, timed, forms);
-    if (!forward || !lane.strings) return;
+    launch(p, lane, in, with_grad, forward, ws, pinned, timed);
+    if (!lane.unsettled) return;
     check(hipEventSynchronize(lane.done), "hipEventSynchronize");
-    bool pairs = false, strings = false;
-    for (size_t i = 0; i < in.size(); ++i) {
-        const bool s = in_string_form(lane.h_flags + FLAG_COUNT * i);
-        strings = strings || s;
-        pairs = pairs || !s;
-    }
-    p->pair_hold = pairs ? kPairHold : std::max(p->pair_hold - 1, 0);
-    const bool missing = (strings && !lane.string_kernels) || (pairs && !lane.pair_kernels);
-    p->pair_run = !strings                    ? p->pair_run + (p->pair_run < kPairRun)
-                  : forms == Forms::pairs     ? -kPairHold
-                                              : std::min(p->pair_run, 0);
-    if (missing) enqueue(p, lane, in, with_grad, forward, ws, pinned, timed);
+    (void)settle(p, lane);
 }
 
 Lane& acquire_lane(vbe_pool* p) {
@@ -1276,16 +1314,14 @@ int pool_launch(vbe_pool* p, int count, const int* slots, const double* const* C
         lane->grad_offsets.push_back(total);
         upload(lane->d_C, lane->h_C, total, lane->stream);
         lane->busy = true;
+        lane->back_src = lane->d_grad;
+        lane->back_dst = lane->h_grad;
+        lane->back_doubles = gradient ? total : 0;
         try {
-            enqueue(p, *lane, in, gradient, true);
-            if (gradient) {
-                check(hipMemcpyAsync(lane->h_grad, lane->d_grad, total * sizeof(double), hipMemcpyDeviceToHost,
-                                     lane->stream),
-                      "gradient D2H");
-                check(hipEventRecord(lane->done, lane->stream), "hipEventRecord");
-            }
+            launch(p, *lane, in, gradient, true);
         } catch (...) {
             (void)hipStreamSynchronize(lane->stream);
+            lane->back_doubles = 0;
             lane->busy = false;
             throw;
         }
@@ -1310,7 +1346,12 @@ int pool_launch_query(vbe_pool* p, int lane, std::string* err) {
         *err = std::string("hipEventQuery: ") + hipGetErrorString(q);
         return -VBE_ERR_DEVICE;
     }
-    return 1;
+    try {
+        return settle(p, p->lanes[lane]) ? 1 : 0;
+    } catch (const std::exception& e) {
+        *err = e.what();
+        return -VBE_ERR_DEVICE;
+    }
 }
 
 int pool_launch_collect(vbe_pool* p, int lane_index, double* energies, double* const* grads, int* status,
@@ -1563,15 +1604,14 @@ int vbe_pool_submit(vbe_pool* pool, int32_t count, const int32_t* slots, const d
         }
         lane.grad_offsets.push_back(total);
         lane.busy = true;
+        lane.back_src = lane.d_grad;
+        lane.back_dst = lane.h_grad;
+        lane.back_doubles = want_gradient ? total : 0;
         try {
-            enqueue(pool, lane, in, want_gradient != 0, true);
-            if (want_gradient)
-                check(hipMemcpyAsync(lane.h_grad, lane.d_grad, total * sizeof(double), hipMemcpyDeviceToHost,
-                                     lane.stream),
-                      "gradient D2H");
-            check(hipEventRecord(lane.done, lane.stream), "hipEventRecord");
+            launch(pool, lane, in, want_gradient != 0, true);
         } catch (...) {
             (void)hipStreamSynchronize(lane.stream);
+            lane.back_doubles = 0;
             lane.busy = false;
             throw;
         }
@@ -1594,7 +1634,7 @@ int vbe_pool_poll(vbe_pool* pool, int32_t ticket, int32_t* done) {
                 return VBE_OK;
             }
             check(q, "hipEventQuery");
-            *done = 1;
+            *done = settle(pool, lane) ? 1 : 0;
             return VBE_OK;
         }
         throw StatusError(VBE_ERR_ARGUMENT, "unknown or already completed ticket");
