@@ -177,7 +177,8 @@ class Waited:
             e = self.pool.evaluate_device([0], c.data_ptr(), g.data_ptr())[0]
             form = self.pool.string_form()[0]
         else:
-            e = self.prob.evaluate_device(c.data_ptr(), g.data_ptr())
+            call = self.prob.evaluate_device_noalloc if self.call == "noalloc" else self.prob.evaluate_device
+            e = call(c.data_ptr(), g.data_ptr())
             form = self.prob.string_form()[0]
         return e, g.cpu().numpy().reshape(C.shape), form
 
@@ -186,7 +187,7 @@ class Waited:
         self.ctx.close()
 
 
-@pytest.mark.parametrize("call", ["evaluate", "two_phase", "device", "pool", "submit", "scheduler"])
+@pytest.mark.parametrize("call", ["evaluate", "two_phase", "device", "noalloc", "pool", "submit", "scheduler"])
 @pytest.mark.parametrize("order", ["ggi", "ggrg", "gggnig", "iiiiiiggi", "rrrrrgg"])
 def test_launches_repeat_with_the_kernels_they_lack(call, order):
     """g: well separated orbitals (string form, after two of them alone); i: ill-conditioned S_act; r: too many rank

@@ -1010,7 +1010,7 @@ __global__ void __launch_bounds__(256) k_string_list_density(const SlotDesc* __r
     for (int i = lane; i < len; i += 64) out[i] = acc[i];
 }
 
-// The listed pairs' response, rows zblocks.. of zpart: workgroup k takes pairs k, k + kStringListRows, ...
+// The listed pairs' response, rows zblocks.. of zpart: workgroup k takes k, k + kStringListRows, ... of them, both ways counted.
 // Both rows of a pair are products of one vector per spin: f = M_a[d_a] M_b[d_b], and sigma = (Ht - E) e is
 // contracted with the other spin's row of M, so that the beta part is the response of the strings
 //   (M_b[d_b][y], t[y]),  t[y] = sum_x M_a[d_a][x] sigma[x][y]
@@ -1031,72 +1031,72 @@ __global__ void __launch_bounds__(256) k_string_list_response(const SlotDesc* __
     string_double4 acc = string_double4{0.0, 0.0, 0.0, 0.0};
     double alpha = 0.0;  // element tid of the alpha part
     const int listed = to_global(sd.flags)[FLAG_DEFERRED];
-    for (int i = blockIdx.x; i < listed; i += gridDim.x) {
+    for (int i = blockIdx.x; i < 2 * listed; i += gridDim.x) {
         int d, e;
-        unpack_pair(to_global(sd.defer)[i], d, e);
+        unpack_pair(to_global(sd.defer)[i >> 1], d, e);
+        if (d == e && (i & 1)) continue;
         double wH, wS;
         pair_weights(sd, topo, d, e, d, e, false, 1.0, wH, wS);
-        for (int way = 0; way < (d == e ? 1 : 2); ++way) {
-            const int bra = way ? e : d, ket = way ? d : e;
-            const int a = t.arank[ket], b = t.brank[ket], A = t.arank[bra], B = t.brank[bra];
-            const uint32_t* ea = t.a.e1 + (size_t)a * Ja;
-            const uint32_t* eb = t.b.e1 + (size_t)b * Jb;
-            const double ma = Ma[(size_t)A * na + a], mb = Mb[(size_t)B * nb + b];
-            __syncthreads();  // the previous pair's rows have been read
-            if (tid < Ja) ua[tid] = signed_value(Ma[(size_t)A * na + (ea[tid] & 0xffff)], ea[tid]);
-            if (tid >= 64 && tid < 64 + Jb) ub[tid - 64] = signed_value(Mb[(size_t)B * nb + (eb[tid - 64] & 0xffff)], eb[tid - 64]);
-            // K = M Ht of the pair, either spin
-            double ka = 0.0, kb = 0.0;
-            for (int x = tid; x < na; x += 256) ka += Ma[(size_t)A * na + x] * Ha[(size_t)x * na + a];
-            for (int y = tid; y <= nb; y += 256) {
-                const double m = y < nb ? Mb[(size_t)B * nb + y] : 0.0, h = y < nb ? Hb[(size_t)y * nb + b] : 0.0;
-                kb += m * h;
-                rows[y] = f64x2{m, wH * ma * h};
-            }
-            if (!t.sym)
-                for (int x = tid; x < na; x += 256) ta[x] = wH * mb * Ha[(size_t)x * na + a];
-            ka = wave_sum(ka);
-            kb = wave_sum(kb);
-            if ((tid & 63) == 0) {
-                part[0][tid >> 6] = ka;
-                part[1][tid >> 6] = kb;
-            }
-            __syncthreads();
-            // opposite spin: wavefront 0 adds the beta targets, 1 the alpha ones (distinct but for the string itself)
-            const bool beta = tid < 64;
-            if (beta || (tid < 128 && !t.sym)) {
-                const int j = tid & 63, J = beta ? Jb : Ja, J2 = beta ? Ja : Jb, noff = beta ? t.b.noff : t.a.noff;
-                double v = 0.0;
-                const uint32_t code = beta ? eb[min(j, J - 1)] : ea[min(j, J - 1)];
-                const int own = (int)(code >> 16 & 0xff);
+        const int bra = i & 1 ? e : d, ket = i & 1 ? d : e;
+        const int a = t.arank[ket], b = t.brank[ket], A = t.arank[bra], B = t.brank[bra];
+        const uint32_t* ea = t.a.e1 + (size_t)a * Ja;
+        const uint32_t* eb = t.b.e1 + (size_t)b * Jb;
+        const double ma = Ma[(size_t)A * na + a], mb = Mb[(size_t)B * nb + b];
+        __syncthreads();  // the previous pair's rows have been read
+        if (tid < Ja) ua[tid] = signed_value(Ma[(size_t)A * na + (ea[tid] & 0xffff)], ea[tid]);
+        if (tid >= 64 && tid < 64 + Jb) ub[tid - 64] = signed_value(Mb[(size_t)B * nb + (eb[tid - 64] & 0xffff)], eb[tid - 64]);
+        // K = M Ht of the pair, either spin
+        double ka = 0.0, kb = 0.0;
+        for (int x = tid; x < na; x += 256) ka += Ma[(size_t)A * na + x] * Ha[(size_t)x * na + a];
+        for (int y = tid; y <= nb; y += 256) {
+            const double m = y < nb ? Mb[(size_t)B * nb + y] : 0.0, h = y < nb ? Hb[(size_t)y * nb + b] : 0.0;
+            kb += m * h;
+            rows[y] = f64x2{m, wH * ma * h};
+        }
+        if (!t.sym)
+            for (int x = tid; x < na; x += 256) ta[x] = wH * mb * Ha[(size_t)x * na + a];
+        ka = wave_sum(ka);
+        kb = wave_sum(kb);
+        if ((tid & 63) == 0) {
+            part[0][tid >> 6] = ka;
+            part[1][tid >> 6] = kb;
+        }
+        __syncthreads();
+        // opposite spin: wavefront 0 adds the beta targets, 1 the alpha ones (distinct but for the string itself)
+        const bool beta = tid < 64;
+        if (beta || (tid < 128 && !t.sym)) {
+            const int j = tid & 63, J = beta ? Jb : Ja, J2 = beta ? Ja : Jb, noff = beta ? t.b.noff : t.a.noff;
+            double v = 0.0;
+            const uint32_t code = beta ? eb[min(j, J - 1)] : ea[min(j, J - 1)];
+            const int own = (int)(code >> 16 & 0xff);
 #pragma unroll 4
-                for (int k = 0; k < J2; ++k) {
-                    const int other = (int)((beta ? ea[k] : eb[k]) >> 16 & 0xff);
-                    v += (beta ? ua[k] : ub[k]) * gt[beta ? other * n2 + own : own * n2 + other];
-                }
-                v = signed_value(wH * v, code);
-                const double itself = wave_sum(j >= noff && j < J ? v : 0.0);
-                if (j < noff) {
-                    if (beta) rows[code & 0xffff][1] += v;
-                    else ta[code & 0xffff] += v;
-                }
-                if (j == 0) {
-                    const double* p = part[beta ? 0 : 1];
-                    const double k = (p[0] + p[1]) + (p[2] + p[3]);
-                    const double s = itself + wH * k + wS * (beta ? ma : mb);
-                    if (beta) rows[b][1] += s;
-                    else ta[a] += s;
-                }
+            for (int k = 0; k < J2; ++k) {
+                const int other = (int)((beta ? ea[k] : eb[k]) >> 16 & 0xff);
+                v += (beta ? ua[k] : ub[k]) * gt[beta ? other * n2 + own : own * n2 + other];
             }
-            __syncthreads();
-            response_products<1>(rows, t.wtab, nb, t.nw, acc);
-            if (!t.sym && tid < n2) {
-                for (int k = 0; k < t.ak; ++k) {
-                    const uint32_t at = t.alist[(size_t)k * n2 + tid];
-                    if (at == ~0u) continue;
-                    const uint32_t code = t.a.e1[at];
-                    alpha += signed_value(Ma[(size_t)A * na + (code & 0xffff)] * ta[at / Ja], code);
-                }
+            v = signed_value(wH * v, code);
+            const double itself = wave_sum(j >= noff && j < J ? v : 0.0);
+            if (j < noff) {
+                if (beta) rows[code & 0xffff][1] += v;
+                else ta[code & 0xffff] += v;
+            }
+            if (j == 0) {
+                const double* p = part[beta ? 0 : 1];
+                const double k = (p[0] + p[1]) + (p[2] + p[3]);
+                const double s = itself + wH * k + wS * (beta ? ma : mb);
+                if (beta) rows[b][1] += s;
+                else ta[a] += s;
+            }
+        }
+        __syncthreads();
+        response_products<1>(rows, t.wtab, nb, t.nw, acc);
+        if (!t.sym && tid < n2) {
+#pragma unroll 8
+            for (int k = 0; k < t.ak; ++k) {
+                const uint32_t entry = t.alist[(size_t)k * n2 + tid], at = entry == ~0u ? 0u : entry;
+                const uint32_t code = t.a.e1[at];
+                const double v = signed_value(Ma[(size_t)A * na + (code & 0xffff)] * ta[at / Ja], code);
+                alpha += entry == ~0u ? 0.0 : v;
             }
         }
     }

@@ -133,7 +133,8 @@ constexpr int kStringPairSegment = 128; // determinants per wavefront of k_strin
 // of 2 pairs listed at 10 orbitals and 20 at 12 to 14. A block the lane kernels keep (condition below
 // kLaneConditionDefault) is never listed; one that may be rank deficient (above kLaneConditionMax) always is.
 constexpr double kStringListError = 1.0e5;
-// Above this many listed pairs a slot stays on the pair kernels: the list costs about 1 us a pair.
+// Above this many listed pairs a slot stays on the pair kernels. A pair costs 2 us in one problem of 12 orbitals (so all of
+// them 0.5 of the 0.65 ms that the strings save there), 6 in one of 14, 0.3 in eight of 12.
 constexpr int kStringListMax = 256;
 constexpr int kStringListRows = 32;     // workgroups (partial rows) of the listed pairs' response
 // Largest |S_act^-1| element (orbitals of unit norm) for which a slot takes the string form.
