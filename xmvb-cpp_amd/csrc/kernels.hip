@@ -812,7 +812,8 @@ struct PartialRows {
     __device__ PartialRows(const SlotDesc& sd, int n_blocks, int begin, int list_rows)
         : rows(n_blocks), list_begin(begin), strings(string_slot(sd)) {
         if (strings) {
-            rows = list_rows + kSingularBlocks;
+            const auto f = to_global(sd.flags);
+            rows = f[FLAG_DEFERRED] == 0 ? 0 : list_rows + (f[FLAG_SINGULAR_PAIRS] ? kSingularBlocks : 0);
             list_begin = 0;
         }
     }

@@ -381,6 +381,7 @@ __global__ void __launch_bounds__(256) k_pairs_singular(const SlotDesc* __restri
     const int n = topo.n, ng = topo.ng, n_det = topo.n_det;
     const int np = n * (n + 1) / 2;
     const int count = to_global(sd.flags)[FLAG_SINGULAR_PAIRS];
+    if (Backward && count == 0 && string_slot(sd)) return;  // k_reduce_partials skips the rows
     extern __shared__ double lds[];
     double* G2 = lds;
     double* sact = G2 + np * np;

@@ -147,30 +147,48 @@ __global__ void __launch_bounds__(256) k_string_minors(const SlotDesc* __restric
 }
 
 // Conditioning of the overlap block of every string pair: 0 where the lane kernels keep it, else the power of
-// two above max|X^-1|, or kMaybeSingular where the complete-pivoting rank rule may call it deficient. One
-// unordered pair per lane, inverted in registers as the lane kernels do. FP64 VALU bound.
-constexpr int kMaybeSingular = 255;
+// two above max|X^-1|, or kMaybeSingular where the complete-pivoting rank rule may call it deficient. Every minor of
+// S_act is at most 1 (Hadamard's bound, orbitals of unit norm), so max|X| max|X^-1| <= 1 / |det X| and only blocks
+// of a small minor are inverted, as the lane kernels do it: a workgroup collects those of its 2,048 unordered
+// pairs, then takes one per lane. 192 problems of 10 orbitals 50 us, 32 of 12 122, one of 14 152 (every block inverted and
+// both triangles written: 129, 500 and 303). Bound by the reads of M and, beyond 12 orbitals, the inversions.
+constexpr int kMaybeSingular = 255, kConditionSteps = 8;
 template <int M>
 __global__ void __launch_bounds__(256) k_string_condition(const SlotDesc* __restrict__ slots, int n, StringSpace sp,
                                                           bool beta) {
     const SlotDesc& sd = slots[blockIdx.z];
     if (!to_global(sd.flags)[FLAG_STRINGS]) return;
     __shared__ double s[kMaxN * kMaxN];
+    __shared__ int small[256 * kConditionSteps], smalls;
     for (int t = threadIdx.x; t < n * n; t += blockDim.x) s[t] = to_global(sd.sact)[t];
+    if (threadIdx.x == 0) smalls = 0;
     __syncthreads();
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)sp.N * (sp.N + 1) / 2) return;
-    int x, y;
-    unpack_pair(t, x, y);
-    LaneBlock<M> b;
-    occupied<M>(sp.mask[x], b.R);
-    occupied<M>(sp.mask[y], b.L);
-    int code = 0;
-    if (!lane_invert<M>(s, n, kLaneConditionDefault, b))  // a NaN counts as singular
-        code = b.cond < kLaneConditionMax ? ilogb(b.inverse) + 1 : kMaybeSingular;
+    const auto minors = to_global(static_cast<const double*>(beta ? sd.sw.Mb : sd.sw.Ma));
     const auto near = to_global(beta ? sd.sw.nearb : sd.sw.neara);
-    near[(size_t)x * sp.N + y] = (unsigned char)code;
-    near[(size_t)y * sp.N + x] = (unsigned char)code;
+    const int pairs = sp.N * (sp.N + 1) / 2;  // at most 5.9 million
+#pragma unroll
+    for (int u = 0; u < kConditionSteps; ++u) {
+        const int t = (blockIdx.x * kConditionSteps + u) * 256 + threadIdx.x;
+        int x, y;
+        unpack_pair(min(t, pairs - 1), x, y);
+        const size_t at = (size_t)y * sp.N + x;  // x <= y, lanes along x
+        const double det = minors[at];
+        if (t >= pairs) continue;
+        if (fabs(det) > 1.01 / kLaneConditionDefault) near[at] = 0;
+        else small[atomicAdd(&smalls, 1)] = t;  // in any order: each is its own element
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < smalls; i += 256) {
+        int x, y;
+        unpack_pair(small[i], x, y);
+        LaneBlock<M> b;
+        occupied<M>(sp.mask[x], b.R);
+        occupied<M>(sp.mask[y], b.L);
+        int code = 0;
+        if (!lane_invert<M>(s, n, kLaneConditionDefault, b))  // a NaN counts as singular
+            code = b.cond < kLaneConditionMax ? ilogb(b.inverse) + 1 : kMaybeSingular;
+        near[(size_t)y * sp.N + x] = (unsigned char)code;
+    }
 }
 
 // Pairs left to the list kernels (kStringListError), flagged per work item of the lane kernels, so that
@@ -187,7 +205,8 @@ __global__ void __launch_bounds__(256) k_string_list(const SlotDesc* __restrict_
          i += (long long)gridDim.x * blockDim.x) {
         int d, e;
         unpack_pair(topo.lane_pairs ? (long long)topo.lane_pairs[i] : i, d, e);
-        const size_t a = (size_t)t.arank[d] * na + t.arank[e], b = (size_t)t.brank[d] * nb + t.brank[e];
+        auto at = [](int x, int y, int N) { return x <= y ? (size_t)y * N + x : (size_t)x * N + y; };
+        const size_t a = at(t.arank[d], t.arank[e], na), b = at(t.brank[d], t.brank[e], nb);
         const int p = max((int)pa[a], (int)pb[b]);
         const bool listed =
             p == kMaybeSingular || (p > 0 && ldexp(fabs(to_global(sd.sw.Ma)[a] * to_global(sd.sw.Mb)[b]), 3 * p) >= limit);
@@ -959,8 +978,8 @@ __global__ void __launch_bounds__(256) k_string_list_density(const SlotDesc* __r
     const StringTopo& t = topo.str;
     const int n = topo.n, n2 = n * n, nc = n * (n - 1) / 2, na = t.a.N, nb = t.b.N;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int item = blockIdx.x * 4 + wave;
-    if (item >= n2 + (t.sym ? 1 : 2) * nc) return;
+    const int item = blockIdx.x * 4 + wave, listed = to_global(sd.flags)[FLAG_DEFERRED];
+    if (listed == 0 || item >= n2 + (t.sym ? 1 : 2) * nc) return;
     const bool opposite = item < n2, alpha = item >= n2 + nc;
     const int L = item - n2 - (alpha ? nc : 0);
     int x = item / n, y = item - x * n;  // opposite spin: y -> x of the alpha string; same spin: the two replaced
@@ -974,7 +993,6 @@ __global__ void __launch_bounds__(256) k_string_list_density(const SlotDesc* __r
     wave_sync();
     const auto Ma = to_global(static_cast<const double*>(sd.sw.Ma)), Mb = to_global(static_cast<const double*>(sd.sw.Mb));
     const StringSpace& own = opposite || alpha ? t.a : t.b;  // the string that the wavefront's item selects
-    const int listed = to_global(sd.flags)[FLAG_DEFERRED];
     for (int i = 0; i < listed; ++i) {
         int d, e;
         unpack_pair(to_global(sd.defer)[i], d, e);
@@ -1018,7 +1036,8 @@ __global__ void __launch_bounds__(256) k_string_list_density(const SlotDesc* __r
 __global__ void __launch_bounds__(256) k_string_list_response(const SlotDesc* __restrict__ slots, TopoDesc topo,
                                                               int zblocks) {
     const SlotDesc& sd = slots[blockIdx.z];
-    if (!string_slot(sd)) return;
+    const int listed = to_global(sd.flags)[FLAG_DEFERRED];
+    if (!string_slot(sd) || (int)blockIdx.x >= 2 * listed) return;  // k_string_gather skips the row
     extern __shared__ __align__(16) double lds[];
     __shared__ double ua[64], ub[64], part[2][4];
     const StringTopo& t = topo.str;
@@ -1030,7 +1049,6 @@ __global__ void __launch_bounds__(256) k_string_list_response(const SlotDesc* __
     const auto gt = to_global(static_cast<const double*>(sd.sw.gt));
     string_double4 acc = string_double4{0.0, 0.0, 0.0, 0.0};
     double alpha = 0.0;  // element tid of the alpha part
-    const int listed = to_global(sd.flags)[FLAG_DEFERRED];
     for (int i = blockIdx.x; i < 2 * listed; i += gridDim.x) {
         int d, e;
         unpack_pair(to_global(sd.defer)[i >> 1], d, e);
@@ -1123,6 +1141,8 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
     const int n = topo.n, n2 = n * n, nc = n * (n - 1) / 2;
     const size_t n4 = (size_t)n2 * n2;
     const auto gp = to_global(static_cast<const double*>(sd.sw.gpart));
+    const int listed = to_global(sd.flags)[FLAG_DEFERRED];  // 0: no listed pairs' chunk
+    const int gchunks = t.gchunks + (listed > 0), wchunks = (t.sym ? 1 : 2) * (t.wchunks + (listed > 0));
     if (bx < tiles) {
         __shared__ double up[kGatherTile][kGatherTile + 1], lo[kGatherTile][kGatherTile + 1];
         int tx, ty;
@@ -1133,7 +1153,7 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
         double v = 0.0, v2 = 0.0;
         const size_t at = (size_t)min(X, n2 - 1) * n2 + min(Y, n2 - 1), at2 = (size_t)min(X2, n2 - 1) * n2 + min(Y2, n2 - 1);
 #pragma unroll 4
-        for (int k = 0; k <= t.gchunks; ++k) {
+        for (int k = 0; k < gchunks; ++k) {
             v += gp[k * n4 + at];
             v2 += gp[k * n4 + at2];
         }
@@ -1149,7 +1169,7 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
             const auto w = to_global(static_cast<const double*>(sd.sw.wpart)) + (size_t)(lb * (lb - 1) / 2 + la) * nc +
                            qb * (qb - 1) / 2 + qa;
             double s = 0.0;
-            for (int k = 0; k < (t.sym ? 1 : 2) * (t.wchunks + 1); ++k) s += w[(size_t)k * nc * nc];
+            for (int k = 0; k < wchunks; ++k) s += w[(size_t)k * nc * nc];
             if (t.sym) s *= 2.0;
             return (q < q2) == (l < l2) ? s : -s;
         };
@@ -1161,21 +1181,22 @@ __global__ void __launch_bounds__(256) k_string_gather(const SlotDesc* __restric
     // dht over both spins: a diagonal of the density counts every electron of the other spin
     for (int X = threadIdx.x; X < n2; X += 256) {
         double va = 0.0, vb = 0.0;
-        for (int k = 0; k <= t.gchunks; ++k)
+        for (int k = 0; k < gchunks; ++k)
             for (int l = 0; l < n; ++l) {
                 va += gp[k * n4 + (size_t)X * n2 + l * (n + 1)];
                 vb += gp[k * n4 + (size_t)l * (n + 1) * n2 + X];
             }
         to_global(sd.sw.hb)[X] = va / t.b.m + vb / t.a.m;
         const auto z = to_global(static_cast<const double*>(sd.sw.zpart));
+        const int zrows = zblocks + min(kStringListRows, 2 * listed);
         double v = 0.0;
 #pragma unroll 8
-        for (int k = 0; k < zblocks; ++k) v += z[(size_t)k * n2 + X];
+        for (int k = 0; k < zrows; ++k) v += z[(size_t)k * n2 + X];
         if (t.sym) v *= 2.0;
         else
             for (int k = 0; k < t.ak; ++k) {
                 const uint32_t at = t.alist[(size_t)k * n2 + X];
-                if (at != ~0u) v += z[(size_t)zblocks * n2 + at];
+                if (at != ~0u) v += z[(size_t)(zblocks + kStringListRows) * n2 + at];
             }
         to_global(sd.sw.Zt)[X] = v;
     }
@@ -1254,7 +1275,7 @@ void minors(hipStream_t st, const SlotDesc* slots, unsigned z, int n, const Stri
     else if (sp.m == M) {
         hipLaunchKernelGGL(k_string_minors<M>, dim3(blocks_for(sp.N), (unsigned)((sp.N + kMinorRows - 1) / kMinorRows), z),
                            dim3(256), 0, st, slots, n, sp, beta);
-        hipLaunchKernelGGL(k_string_condition<M>, dim3(blocks_for((long long)sp.N * (sp.N + 1) / 2), 1, z), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_string_condition<M>, dim3(blocks_for((long long)sp.N * (sp.N + 1) / 2, 256 * kConditionSteps), 1, z), dim3(256), 0, st,
                            slots, n, sp, beta);
     } else minors<M + 1>(st, slots, z, n, sp, beta);
 }
@@ -1365,7 +1386,7 @@ void launch_string_forward(hipStream_t st, const SlotDesc* slots, unsigned z, co
 void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, const TopoDesc& topo) {
     const StringTopo& t = topo.str;
     const int n = topo.n, n2 = n * n, nc = n * (n - 1) / 2, na = t.a.N, nb = t.b.N;
-    const int wc = t.wchunks, zb = z_blocks(t), zrows = zb + kStringListRows;
+    const int wc = t.wchunks, zb = z_blocks(t);
     const dim3 w_grid((unsigned)((nc * wc + 3) / 4), 1, z);
     const int ti = (na + kProductTile - 1) / kProductTile, tj = (nb + kProductTile - 1) / kProductTile;
     const int row_waves = nb > 1000 ? 2 : 4;  // two wavefronts' rows of 3432 strings leave two workgroups per CU
@@ -1398,7 +1419,7 @@ void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, c
         if (!t.sym) {
             if (wc > 0) hipLaunchKernelGGL(k_string_same<true>, w_grid, dim3(256), 0, st, slots, topo, s, wc, add);
             hipLaunchKernelGGL(k_string_response_alpha, dim3((unsigned)na, 1, z), dim3(256), sizeof(double) * nb, st, slots,
-                               topo, zrows * n2, add);
+                               topo, (zb + kStringListRows) * n2, add);
         }
     }
     hipLaunchKernelGGL(k_string_list_density, dim3((unsigned)((n2 + (t.sym ? 1 : 2) * nc + 3) / 4), 1, z), dim3(256), 0, st,
@@ -1407,7 +1428,7 @@ void launch_string_backward(hipStream_t st, const SlotDesc* slots, unsigned z, c
                        sizeof(double) * std::max<size_t>(2 * (nb + 1) + (t.sym ? 0 : na), 4 * 256), st, slots, topo, zb);
     const long long n4 = (long long)n2 * n2;
     const int gt = (n2 + kGatherTile - 1) / kGatherTile, gtiles = gt * (gt + 1) / 2;
-    hipLaunchKernelGGL(k_string_gather, dim3((unsigned)gtiles + 1, 1, z), dim3(256), 0, st, slots, topo, gtiles, zrows);
+    hipLaunchKernelGGL(k_string_gather, dim3((unsigned)gtiles + 1, 1, z), dim3(256), 0, st, slots, topo, gtiles, zb);
     const unsigned vb = blocks_for(n4);
     hipLaunchKernelGGL(k_string_pullback, dim3(vb + n2, 1, z), dim3(256), 0, st, slots, n, (int)vb);
     hipLaunchKernelGGL(k_string_adjoint, dim3(blocks_for(topo.ng + 2 * n2), 1, z), dim3(256), 0, st, slots, n, topo.ng);

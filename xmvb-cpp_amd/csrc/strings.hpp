@@ -105,7 +105,7 @@ struct StringWork {
     double *Ma, *Mb;     // minors of S_act over all string pairs
     double *Ja, *Jb;     // sum over the occupied l2 of gt[q n + l][l2 l2], per string
     double *Ha, *Hb;     // same-spin Hamiltonian in the dual frame, [x][a]
-    unsigned char *neara, *nearb;  // string pairs: conditioning of the overlap block (k_string_condition)
+    unsigned char *neara, *nearb;  // string pairs: conditioning of the overlap block, [y][x] for x <= y (k_string_condition)
     double *Ka, *Kb;     // same-spin Hamiltonian between strings; during the forward, over gpart and on
     double *gpart, *wpart, *zpart;
     double *gs, *hb, *V, *W2, *Zt;
