@@ -203,7 +203,10 @@ int vbe_last_error(const vbe_context* ctx, char* buf, size_t len);
  * reference (below 1e9 a row-pivoted block is provably full rank under that rule); 0 sends every
  * pair through the complete-pivoting path. Default 1e5: worse-conditioned blocks then follow the
  * reference's pivot order, which keeps their rounding close to it; at the default the pairs may also
- * be evaluated over determinant strings where S_act is well conditioned. Applies to later evaluations.
+ * be evaluated over determinant strings where S_act is well conditioned, but for those whose inverse form
+ * loses digits, so that the gradient of either form agrees with the other's to 1e-9 of its norm. (With a block
+ * of smallest singular value 1e-8 the inverse form itself is exact to 7e-8, at 1e-10 to 8e-4.) Applies to later
+ * evaluations.
  * No counterpart in the reference, which has a single (CPU) pair path. */
 int vbe_set_pair_condition_limit(vbe_context* ctx, double limit);
 /* Storage precision of the RI factors for problems and pools created after the call

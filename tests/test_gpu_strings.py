@@ -341,7 +341,7 @@ def test_selected_states(kw, n_act, mult, states):
 
 
 def test_string_arrays_give_way_to_slots():
-    """Two slots of 12 orbitals (30 MB of string arrays each) under budgets that leave out the arrays of one and of both:
+    """Two slots of 12 orbitals (24 MB of string arrays each) under budgets that leave out the arrays of one and of both:
     the slots load as they would without the string form, and the pair kernels serve what has none."""
     topo = vb.Topology.build("COV", 12, 12, 1)
     sps = [vb.synthetic_problem(70 + k, 30, 12, 45) for k in range(2)]
